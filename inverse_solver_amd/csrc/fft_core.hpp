@@ -33,6 +33,15 @@ __device__ __forceinline__ float2 cconj(float2 a) { return make_float2(a.x, -a.y
 __device__ __forceinline__ float2 cmul_mi(float2 a) { return make_float2(a.y, -a.x); }
 __device__ __forceinline__ float2 cmul_pi(float2 a) { return make_float2(-a.y, a.x); }
 
+// Barrier for data exchanged through LDS.  __syncthreads() orders global memory too: it waits
+// for every load in flight, so operands requested ahead of a phase would be waited for at its
+// first barrier.  This one waits for the LDS operations alone.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---------------------------------------------------------------- compile-time trig
 constexpr double kPi = 3.14159265358979323846264338327950288;
 

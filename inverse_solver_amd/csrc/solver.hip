@@ -1770,12 +1770,12 @@ struct Solver {
     return best;
   }
 
-  DevBuf<float2> tv_in, tv_y, tv_P, tv_R;   // used as float arrays for real input
+  DevBuf<float2> tv_in, tv_y, tv_P;   // used as float arrays for real input
   DevBuf<float2> gr_u, gr_w;
   DevBuf<double2> gr_out;
 
   // Both element types share the buffers: a real problem of n voxels uses the first
-  // n (or 3n) floats of buffers sized for n complex values.
+  // n (or 9n) floats of buffers sized for n complex values.
   void tv_prox(const void* in, void* out, const uint32_t* dims, double lam, double vmin, double vmax,
                double vimag_max, int non_neg, int dirichlet, uint32_t inner, int mem, bool cplx) {
     require(in && out && dims, CBS_ERR_ARG, "null TV argument");
@@ -1786,8 +1786,7 @@ struct Solver {
     const size_t esz = cplx ? sizeof(float2) : sizeof(float);
     const long long nf = cplx ? 2 * n : n;   // floats per volume
     tv_y.ensure((size_t)n);
-    tv_P.ensure((size_t)(3 * n));
-    tv_R.ensure((size_t)(3 * n));
+    tv_P.ensure((size_t)(9 * n));   // P_{k-1}, P_k and P_{k+1}
     const void* din = in;
     if (mem == CBS_MEM_HOST) {
       tv_in.ensure((size_t)n);
@@ -1799,32 +1798,33 @@ struct Solver {
     a.lam = (float)lam; a.vmin = (float)vmin; a.vmax = (float)vmax;
     a.vimag_max = (vimag_max > 0) ? (float)vimag_max : 0.f;   // NaN or <= 0: no cap (the reference tests > 0)
     a.non_neg = non_neg; a.dirichlet = dirichlet;
-    float* P = reinterpret_cast<float*>(tv_P.p);
-    float* R = reinterpret_cast<float*>(tv_R.p);
+    float* Pk[3];
+    for (int k = 0; k < 3; ++k) Pk[k] = reinterpret_cast<float*>(tv_P.p) + (size_t)k * 3 * nf;
     float* Y = reinterpret_cast<float*>(tv_y.p);
-    hipLaunchKernelGGL(tv_zero, dim3(grid_for(3 * nf)), dim3(256), 0, stream, P, 3 * nf);
-    hipLaunchKernelGGL(tv_zero, dim3(grid_for(3 * nf)), dim3(256), 0, stream, R, 3 * nf);
+    if (inner == 0) hipLaunchKernelGGL(tv_zero, dim3(grid_for(3 * nf)), dim3(256), 0, stream, Pk[0], 3 * nf);
     const unsigned g = grid_for(n);
-    auto div_project = [&](const float* Q, void* dst) {
-      if (cplx)
-        hipLaunchKernelGGL(tv_div_project_c, dim3(g), dim3(256), 0, stream, (const float2*)din, (const float2*)Q,
-                           (float2*)dst, a);
-      else
-        hipLaunchKernelGGL(tv_div_project, dim3(g), dim3(256), 0, stream, (const float*)din, Q, (float*)dst, a);
-    };
+    int cur = 0;                // P_k in Pk[cur], P_{k-1} in the one before it
     double t = 1.0;
+    float theta = 0.f;          // the momentum between P_k and P_{k-1}
     for (uint32_t it = 0; it < inner; ++it) {
       const double tn = (1.0 + std::sqrt(1.0 + 4.0 * t * t)) / 2.0;
-      const float theta = (float)((t - 1.0) / tn);
-      div_project(R, Y);
+      // theta is 0 after the first iteration: P_1 stands in for the P_0 = 0 that no buffer holds
+      const int nxt = (cur + 1) % 3, prv = it == 1 ? cur : (cur + 2) % 3;
       if (cplx)
-        hipLaunchKernelGGL(tv_dual_update_c, dim3(g), dim3(256), 0, stream, (const float2*)Y, (float2*)P,
-                           (float2*)R, a, theta);
+        tv_inner_complex(stream, (const float2*)din, (const float2*)Pk[cur], (const float2*)Pk[prv], (float2*)Pk[nxt],
+                         a, theta, it == 0);
       else
-        hipLaunchKernelGGL(tv_dual_update, dim3(g), dim3(256), 0, stream, (const float*)Y, P, R, a, theta);
+        tv_inner_real(stream, (const float*)din, Pk[cur], Pk[prv], Pk[nxt], a, theta, it == 0);
+      theta = (float)((t - 1.0) / tn);
       t = tn;
+      cur = nxt;
     }
-    div_project(P, mem == CBS_MEM_HOST ? (void*)Y : out);
+    void* dst = mem == CBS_MEM_HOST ? (void*)Y : out;
+    if (cplx)
+      hipLaunchKernelGGL(tv_div_project_c, dim3(g), dim3(256), 0, stream, (const float2*)din, (const float2*)Pk[cur],
+                         (float2*)dst, a);
+    else
+      hipLaunchKernelGGL(tv_div_project, dim3(g), dim3(256), 0, stream, (const float*)din, Pk[cur], (float*)dst, a);
     HIP_CHECK(hipGetLastError());
     if (mem == CBS_MEM_HOST) HIP_CHECK(hipMemcpyAsync(out, Y, (size_t)n * esz, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));

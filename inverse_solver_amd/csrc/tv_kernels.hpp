@@ -9,16 +9,18 @@ struct TvArgs {
   int non_neg, dirichlet;
 };
 
-// Real potential (kappamax = 0): one float per voxel; the dual P, R hold 3 * n floats.
+// y = project(in - lam div(Q)) of a real potential (one float per voxel, the dual Q three) or a
+// complex one (complex64 per voxel).
 __global__ void tv_div_project(const float* __restrict__ in, const float* __restrict__ Q, float* __restrict__ y,
                                TvArgs a);
-__global__ void tv_dual_update(const float* __restrict__ y, float* __restrict__ P, float* __restrict__ R, TvArgs a,
-                               float theta);
-// Complex potential: complex64 per voxel; the dual holds 3 * n complex values.
 __global__ void tv_div_project_c(const float2* __restrict__ in, const float2* __restrict__ Q, float2* __restrict__ y,
                                  TvArgs a);
-__global__ void tv_dual_update_c(const float2* __restrict__ y, float2* __restrict__ P, float2* __restrict__ R,
-                                 TvArgs a, float theta);
+// One inner iteration: Pn = P_{k+1} from Pc = P_k and Pp = P_{k-1} (three volumes each, Pn apart
+// from both) and the momentum theta between them; first: P_0 = 0, Pc and Pp are not read.
+void tv_inner_real(hipStream_t st, const float* in, const float* Pc, const float* Pp, float* Pn, const TvArgs& a,
+                   float theta, bool first);
+void tv_inner_complex(hipStream_t st, const float2* in, const float2* Pc, const float2* Pp, float2* Pn,
+                      const TvArgs& a, float theta, bool first);
 __global__ void tv_zero(float* __restrict__ buf, long long n);
 
 // Misfit gradient from the forward and adjoint 3D fields (n_rhs blocks of nx*ny*nz complex64).
