@@ -767,8 +767,9 @@ __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb
   __shared__ float2 lds[N * T];
   __shared__ float2 s_tw[N];
   const int ntile = (c.nx + T - 1) / T;
-  const int xt = blockIdx.x % ntile;
-  const int o = blockIdx.x / ntile;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks
   if (cv.norms && conv_stopped(cv, jj - 1, slot)) return;
   const int flip = flip_of(jj, parity, slot);
@@ -844,8 +845,9 @@ __global__ __launch_bounds__(NT) void fft_strided(float2* data, int nx, long lon
   __shared__ float2 s_tw[N];   // twiddles: a task's R1 - 1 of them differ from lane to lane
   for (int i = threadIdx.x; i < N; i += NT) s_tw[i] = tw[i];
   const int ntile = (nx + T - 1) / T;
-  const int xt = blockIdx.x % ntile;
-  const int o = blockIdx.x / ntile;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
   const int tvalid = nx - xt * T < T ? nx - xt * T : T;
   float2* base = data + (long long)(o / inner) * os2 + (long long)(o % inner) * os + (long long)xt * T;
   auto ad = [](int l, int e) { return e * T + l; };

@@ -114,8 +114,9 @@ __global__ __launch_bounds__(NT) void blue_strided(float2* data, int nx, long lo
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (nx + T - 1) / T;
-  const int xt = blockIdx.x % ntile;
-  const int o = blockIdx.x / ntile;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
   if (o >= nouter) return;
   const int tv = nx - xt * T < T ? nx - xt * T : T;
   float2* base = data + (long long)(o / inner) * os2 + (long long)(o % inner) * os + (long long)xt * T;
@@ -303,8 +304,9 @@ __global__ __launch_bounds__(NT) void blue_strided_green(float2* data, Tables tb
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (c.nx + T - 1) / T;
-  const int xt = blockIdx.x % ntile;
-  const int o = blockIdx.x / ntile;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks
   if (cv.norms && conv_stopped(cv, jj - 1, slot)) return;
   const int flip = flip_of(jj, parity, slot);

@@ -154,8 +154,9 @@ __global__ void fft_strided_rt(float2* data, int nx, long long es, long long os,
   float2* a = rt_lds;
   float2* b = rt_lds + (long long)T * L;
   const int ntile = (nx + T - 1) / T;
-  const int xt = blockIdx.x % ntile;
-  const int o = blockIdx.x / ntile;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
   if (o >= nouter) return;
   const int tv = nx - xt * T < T ? nx - xt * T : T;
   float2* base = data + (long long)(o / inner) * os2 + (long long)(o % inner) * os + (long long)xt * T;

@@ -90,13 +90,6 @@ __device__ __forceinline__ float tv_rsqrt(float s) {
   return s < 3.0e38f ? fmaf(0.5f * r, e, r) : r;
 }
 
-// Position of block b of nb in an order that gives each of the 8 XCDs (blocks go to them round
-// robin) a contiguous eighth.
-__device__ __forceinline__ unsigned xcd_position(unsigned b, unsigned nb) {
-  const unsigned q = nb / 8, r = nb % 8, k = b % 8;
-  return k * q + min(k, r) + b / 8;
-}
-
 template <class T, int ZC, bool FIRST, class Off>
 __global__ __launch_bounds__(kTvX * kTvY) void tv_inner(const T* __restrict__ in, const T* __restrict__ Pc,
                                                         const T* __restrict__ Pp, T* __restrict__ Pn, TvArgs a,
