@@ -1,7 +1,7 @@
 // Line FFTs of any length, planned at run time (the per-axis form and the 2D
 // convolution-grid transforms of grids whose line lengths have no compiled kernel).
 //
-// A length n = product of radices from {2, 3, 4, 5, 7, 8, 9, 11, 13, 16} runs as a
+// Lengths up to 448 run as products with the DFT matrix (fft_dense.hip).  Above, a length n = product of radices from {2, 3, 4, 5, 7, 8, 9, 11, 13, 16} runs as a
 // mixed-radix Stockham transform (natural order in and out) in LDS, one stage per
 // radix, ping-ponging between two LDS buffers.  Any other n (a prime factor above 13)
 // runs as Bluestein's chirp-z transform: x_n conj(c_n), c_n = exp(i pi n^2 / n), is
@@ -54,6 +54,37 @@ struct BlueArgs {
   const float2* bpos;       // [L] DFT_L of the chirp filter over L, in the forward output order of L
   const float2* tw;         // [L] exp(-2 pi i e / L)
 };
+// Line transforms as products with the DFT matrix on the matrix cores (fft_dense.hip): n = F m,
+// an m-point product for every residue class and F-point butterflies.
+struct DenseArgs {
+  int n, F, m;
+  int ks;                   // steps of 4 elements up to floor(m / 2)
+  int ntask;                // F x blocks of 16 rows up to floor(m / 2)
+  int inv_F;                // ceil(65536 / F): task / F = task inv_F >> 16
+  float inv_m;              // 1 / m
+  const float2* tab;        // [m] (cos, sin)(2 pi e / m), then [n] exp(-2 pi i e / n)
+};
+// values of the tables a block holds
+__host__ __device__ inline int dense_tables(const DenseArgs& a) { return a.m + (a.F > 1 ? a.n : 0); }
+using DenseRowsFn = void (*)(float2*, long long, DenseArgs, int);
+using DenseStridedFn = void (*)(float2*, int, long long, long long, int, DenseArgs, int, int, long long);
+using DenseRowsUpdateFn = void (*)(StateArgs, Tables, Consts, DenseArgs, int, int, int, int, ConvArgs);
+using DenseStridedGreenFn = void (*)(float2*, Tables, Consts, DenseArgs, const uint8_t*, int, ConvArgs);
+struct DenseInfo {
+  DenseRowsFn rows;
+  DenseStridedFn strided;
+  DenseRowsUpdateFn rows_update[3];   // any launch; steady UPD_DEFER; steady UPD_PAIR
+  DenseStridedGreenFn strided_green;
+  int nmax, tasks;          // longest line, most tasks of a tile
+  int nt_rows, nt_strided;  // threads of a block
+  int lines;                // lines of a tile
+  // dynamic LDS: the tables and the tile (rows: one word of padding an element)
+  size_t lds_rows(const DenseArgs& a) const { return (size_t)(a.n * (lines + 1) + dense_tables(a)) * sizeof(float2); }
+  size_t lds_strided(const DenseArgs& a) const { return (size_t)(a.n * lines + dense_tables(a)) * sizeof(float2); }
+};
+// the kernels for lines of n elements and ntask tasks (null: too long)
+const DenseInfo* find_dense(int n, int ntask);
+
 // rows: NL contiguous lines of n per block; strided: as fft_strided_rt with T = t lines
 using BlueRowsFn = void (*)(float2*, long long, BlueArgs, int);
 using BlueStridedFn = void (*)(float2*, int, long long, long long, int, BlueArgs, int, int, long long);

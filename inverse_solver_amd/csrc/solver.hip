@@ -137,6 +137,8 @@ struct RtPlan {
   const BlueInfo* bi = nullptr;   // Bluestein on a compiled convolution length (else k)
   BlueArgs ba{};
   int pref = 0;                   // built with prefer_blue
+  const DenseInfo* di = nullptr;  // products with the DFT matrix (else bi or k)
+  DenseArgs da{};
 };
 
 // Stage radices of a Stockham transform of length L (16, 8, 4, 2 for the power of two,
@@ -162,7 +164,29 @@ static int smooth_at_least(int m) {
   }
 }
 
-// Plan of the length-n line transform: Stockham when n factors into the radices,
+// Split n = F m of the matrix-core transform (fft_dense.hip) that takes the fewest cycles of a
+// SIMD for 16 lines: 4 x 32 a matrix step, 4 a vector instruction (about 12 an element for the
+// butterfly's LDS traffic and twiddle, and its additions).
+static void dense_split(int n, DenseArgs& a) {
+  double best = 0.0;
+  for (int F = 1; F <= 8; ++F) {
+    if (n % F) continue;
+    const int m = n / F, h = m / 2, ks = h / 4 + 1, rt = h / 16 + 1;
+    const double bf = F == 1 ? 0.0 : n * (12.0 + (F == 7 ? 2.0 * F : 3.0 * std::log2((double)F)));
+    const double cost = 128.0 * F * rt * ks + bf;
+    if (a.n == 0 || cost < best) {
+      best = cost;
+      a.n = n;
+      a.F = F;
+      a.m = m;
+      a.ks = ks;
+      a.ntask = F * rt;
+    }
+  }
+}
+
+// Plan of the length-n line transform: products with the DFT matrix on the matrix cores up to
+// the lengths fft_dense.hip holds; above, Stockham when n factors into the radices,
 // else Bluestein with the chirp c_k = exp(i pi k^2 / n) and the DFT of the chirp
 // filter over a length L >= 2n - 1 (FP64 on the host, rounded to complex64) -- on the
 // shortest compiled convolution length when one is long enough (fft_blue.hip), else
@@ -175,7 +199,27 @@ static void build_rt(RtPlan& P, int n, bool prefer_blue = false) {
   std::vector<int> rs;
   int L = n, blue = 0;
   P.bi = nullptr;
+  P.di = nullptr;
   P.pref = prefer_blue ? 1 : 0;
+  DenseArgs da{};
+  dense_split(n, da);
+  P.di = find_dense(n, da.ntask);
+  if (P.di) {
+    P.k = RtFft{};
+    P.k.n = n;
+    std::vector<float2> tab(da.m), tn = twiddles(n);
+    for (int e = 0; e < da.m; ++e) {
+      const double ang = 2.0 * M_PI * (double)e / (double)da.m;
+      tab[e] = make_float2((float)std::cos(ang), (float)std::sin(ang));
+    }
+    tab.insert(tab.end(), tn.begin(), tn.end());
+    P.tw.upload(tab);
+    da.tab = P.tw.p;
+    da.inv_F = (65536 + da.F - 1) / da.F;
+    da.inv_m = 1.0f / (float)da.m;
+    P.da = da;
+    return;
+  }
   if (!rt_factor(n, rs) || (prefer_blue && find_blue(2 * n - 1))) {
     blue = 1;
     P.bi = find_blue(2 * n - 1);
@@ -339,6 +383,13 @@ struct Solver {
   RtPlan rtp[3], io_rtx, io_rty;
 
   void rt_rows(const RtPlan& P, float2* data, long long nrows, int inverse) {
+    if (P.di) {
+      const long long nblk = (nrows + P.di->lines - 1) / P.di->lines;
+      require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
+      timed(2, [&] { hipLaunchKernelGGL(P.di->rows, dim3((unsigned)nblk), dim3(P.di->nt_rows), P.di->lds_rows(P.da), stream,
+                                        data, nrows, P.da, inverse); });
+      return;
+    }
     if (P.bi) {
       const long long nblk = (nrows + P.bi->nl - 1) / P.bi->nl;
       require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
@@ -357,6 +408,14 @@ struct Solver {
   void rt_strided(const RtPlan& P, float2* data, int ncols, long long es, long long os, long long nouter,
                   int inverse, long long inner = 0, long long os2 = 0) {
     const int in = (int)(inner > 0 ? inner : nouter);
+    if (P.di) {
+      const long long nblk = (long long)((ncols + P.di->lines - 1) / P.di->lines) * nouter;
+      require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
+      timed(2, [&] { hipLaunchKernelGGL(P.di->strided, dim3((unsigned)nblk), dim3(P.di->nt_strided),
+                                        P.di->lds_strided(P.da), stream, data, ncols, es, os, (int)nouter, P.da,
+                                        inverse, in, os2); });
+      return;
+    }
     if (P.bi) {
       const int T = P.bi->t;
       const long long nblk = (long long)((ncols + T - 1) / T) * nouter;
@@ -477,7 +536,8 @@ struct Solver {
       p.form = CBS_FORM_PLAIN;         // grids without either run the per-axis form
     }
     // per-axis form: compiled line FFTs where the length has one, run-time-planned
-    // (Stockham, or Bluestein for prime factors above 13) for every other length
+    // (matrix-core products, above 448 points Stockham, or Bluestein for prime factors above 13)
+    // for every other length
     p.rw = find_fft_rows(nx);
     p.sy = find_fft_strided(ny, 0);
     p.sz = find_fft_strided(nz, 0);
@@ -486,11 +546,11 @@ struct Solver {
     p.rt[2] = !p.sz;
     const int dims[3] = {nx, ny, nz};
     // one-component runs fuse the x transforms with the update and the z transforms with
-    // the Green's multiply when they are compiled (line FFT or Bluestein on a compiled
-    // convolution length), so those two axes take Bluestein's transform over run-time
-    // stages (12-rhs solves on 169^2 x 75, 98^2 x 90, 126^2 x 78 and 147^2 x 77 grids: 22.0,
-    // 22.4, 17.1 and 17.5 -> 25.0, 29.3, 26.8 and 22.4 Gvoxel-iter/s); y, which no pass
-    // fuses, keeps the run-time stages
+    // the Green's multiply where a fused kernel holds the length: the compiled line FFTs, the
+    // matrix-core transforms (up to 448 points), and above those Bluestein's transform on a compiled
+    // length, which x and z therefore prefer to run-time stages there (fused kernels took 169^2 x
+    // 75, 98^2 x 90, 126^2 x 78 and 147^2 x 77 grids of 12 rhs, then on Bluestein's transform, from
+    // 22.0, 22.4, 17.1 and 17.5 to 25.0, 29.3, 26.8 and 22.4 Gvoxel-iter/s)
     const bool fuse = P == 1 && p.form == CBS_FORM_PLAIN;
     for (int j = 0; j < 3; ++j) {
       const int pref = fuse && j != 1 ? 1 : 0;
@@ -902,19 +962,21 @@ struct Solver {
       else if (axis == 1) fy();
       else fz();
     };
-    // single-component runs whose x (z) lines are Bluestein-transformed on a compiled
-    // length: the x inverse, the update and the x forward (the z forward, the Green's
-    // multiply and the z inverse) run as one launch each
-    // (on a compiled line length, the compiled fused passes of lines_fused_inst.hip)
+    // single-component runs: the x inverse, the update and the x forward (the z forward, the
+    // Green's multiply and the z inverse) run as one launch each, on compiled line lengths
+    // (lines_fused_inst.hip), matrix-core products (fft_dense.hip) or Bluestein's transform on a
+    // compiled length (fft_blue.hip)
     const bool fuse = P == 1 && plan.form == CBS_FORM_PLAIN;   // CBS_FORM_AXES: every pass on its own
     const BlueInfo* bx = (fuse && plan.rt[0]) ? rtp[0].bi : nullptr;
     const BlueInfo* bz = (fuse && plan.rt[2]) ? rtp[2].bi : nullptr;
+    const DenseInfo* dx = (fuse && plan.rt[0]) ? rtp[0].di : nullptr;
+    const DenseInfo* dz = (fuse && plan.rt[2]) ? rtp[2].di : nullptr;
     const RowsUpdateInfo* cx = (fuse && !plan.rt[0]) ? find_rows_update(nx) : nullptr;
     const StridedGreenInfo* cz = (fuse && !plan.rt[2]) ? find_strided_green(nz) : nullptr;
     const long long rows = (long long)ny * nz;
     require(rows < (1ll << 31), CBS_ERR_UNSUPPORTED, "grid too large for the per-axis passes");
     auto xpass = [&](int upd, int fwd, int jj_inv, int jj_fwd) {   // (x inverse,) update(, x forward)
-      if (!bx && !cx) {
+      if (!bx && !cx && !dx) {
         if (upd != UPD_NONE) fft1(0, 1);
         update(upd, fwd, jj_inv, jj_fwd);
         if (fwd != FWD_NONE) fft1(0, 0);
@@ -923,9 +985,13 @@ struct Solver {
       StateArgs s = state_args(1);
       s.norms = norm_row(jj_inv, nv);
       if (conv_tol > 0.0 && upd == UPD_VQ_ADD) s.fref = ws.fref;
-      const int nl = bx ? bx->nl : cx->rows;
+      const int nl = dx ? dx->lines : bx ? bx->nl : cx->rows;
       const dim3 g((unsigned)((rows + nl - 1) / nl), (unsigned)nv);
-      if (bx)
+      const int steady = fwd != FWD_GAMMA ? 0 : upd == UPD_DEFER ? 1 : upd == UPD_PAIR ? 2 : 0;
+      if (dx)
+        timed(2, [&] { hipLaunchKernelGGL(dx->rows_update[steady], g, dim3(dx->nt_rows), dx->lds_rows(rtp[0].da), stream, s, tb, c,
+                                          rtp[0].da, upd, fwd, jj_inv, jj_fwd, cv); });
+      else if (bx)
         timed(2, [&] { hipLaunchKernelGGL(bx->rows_update, g, dim3(bx->nt), 0, stream, s, tb, c, rtp[0].ba, upd, fwd,
                                           jj_inv, jj_fwd, cv); });
       else
@@ -938,6 +1004,14 @@ struct Solver {
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
         timed(2, [&] { hipLaunchKernelGGL(cz->fn, dim3((unsigned)nblk), dim3(cz->nt), 0, stream, ws.spec, tb, c,
                                           tabs.tw_z.p, ws.parity, jj, cv); });
+        return;
+      }
+      if (dz) {
+        const long long nblk = (long long)((nx + dz->lines - 1) / dz->lines) * ny * nv;
+        require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
+        timed(2, [&] { hipLaunchKernelGGL(dz->strided_green, dim3((unsigned)nblk), dim3(dz->nt_strided),
+                                          dz->lds_strided(rtp[2].da), stream, ws.spec, tb, c, rtp[2].da, ws.parity, jj,
+                                          cv); });
         return;
       }
       if (!bz) {
