@@ -307,6 +307,14 @@ int cbs_get_norms(cbs_handle h, double* out, uint32_t n_rhs, uint32_t n_iter);
  * default) turns it off.  Norms are then tracked as with track_norms. */
 int cbs_set_convergence(cbs_handle h, double tol);
 
+/* Transforms of line lengths without a compiled FFT (prime factors above 5), in the per-axis form and
+ * the 2D grids.  CBS_TRANSFORMS_FASTEST (the default): the matrix-core products up to 448 points.
+ * CBS_TRANSFORMS_FIXED: Bluestein's transform and the run-time stages, whose rounding does not
+ * change with the library: for callers that compare results bit for bit with earlier ones, as
+ * BACKWARD_SOLVER_MULTI's FP64 gradient is.  No counterpart in the reference, which plans cuFFT. */
+enum { CBS_TRANSFORMS_FASTEST = 0, CBS_TRANSFORMS_FIXED = 1 };
+int cbs_set_transforms(cbs_handle h, int kind);
+
 /* Iterations each rhs of the last solve ran (Bornmax unless the convergence test
  * stopped it earlier): out[r], r < n_rhs, n_rhs equal to the last solve's. */
 int cbs_get_iterations(cbs_handle h, uint32_t* out, uint32_t n_rhs);

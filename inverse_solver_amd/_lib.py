@@ -14,6 +14,7 @@ LIB_PATH = os.path.join(_HERE, 'libcbs_hip.so')
 
 CBS_OK, CBS_ERR_ARG, CBS_ERR_HANDLE, CBS_ERR_HIP, CBS_ERR_UNSUPPORTED, CBS_ERR_STATE, CBS_ERR_MEMORY = range(7)
 CBS_MEM_HOST, CBS_MEM_DEVICE = 0, 1
+CBS_TRANSFORMS_FASTEST, CBS_TRANSFORMS_FIXED = 0, 1
 CBS_FORM_FUSED, CBS_FORM_PLAIN, CBS_FORM_ROWS, CBS_FORM_AXES = 0, 1, 2, 3
 
 EXPORTED = [
@@ -24,7 +25,8 @@ EXPORTED = [
     'cbs_footprint', 'cbs_get_plan', 'cbs_autotune', 'cbs_tv_prox', 'cbs_tv_prox_complex', 'cbs_field_gradient',
     'cbs_phase_residues', 'cbs_phase_integrate', 'cbs_phase_branch_cuts', 'cbs_phase_unwrap',
     'cbs_set_convergence', 'cbs_get_iterations', 'cbs_solve_3d_noalloc', 'cbs_fista_prox_input',
-    'cbs_fista_momentum', 'cbs_field_pupil', 'cbs_solve_field', 'cbs_last_error', 'cbs_abi_version',
+    'cbs_fista_momentum', 'cbs_field_pupil', 'cbs_solve_field', 'cbs_set_transforms', 'cbs_last_error',
+    'cbs_abi_version',
 ]
 
 
@@ -89,6 +91,7 @@ def _load():
         'cbs_phase_unwrap': ([i32, vp, vp, C.POINTER(C.c_uint32), i32], i32),
         'cbs_set_convergence': ([vp, C.c_double], i32),
         'cbs_solve_3d_noalloc': ([vp, vp, u32, vp], i32),
+        'cbs_set_transforms': ([vp, i32], i32),
         'cbs_get_iterations': ([vp, C.POINTER(C.c_uint32), u32], i32),
         'cbs_fista_prox_input': ([vp, vp, vp, C.c_double, C.c_uint64, i32, vp], i32),
         'cbs_fista_momentum': ([vp, vp, i32, vp, vp, vp, C.c_uint64, C.c_double, C.c_double], i32),

@@ -14,6 +14,7 @@ import time
 
 import numpy as np
 
+from ._lib import CBS_TRANSFORMS_FIXED, check, lib
 from .forward_solver import FORWARD_SOLVER_CONVERGENT_BORN, get_default_parameters as fwd_defaults
 from .params import update_struct
 from .tv import tv_fista_inner
@@ -45,6 +46,10 @@ class BACKWARD_SOLVER_MULTI:
         fp['return_reflection'] = False          # the gradient reads only the transmitted and 3D fields
         self.forward = FORWARD_SOLVER_CONVERGENT_BORN(fp, device=device, options=options)
         self.adjoint = FORWARD_SOLVER_CONVERGENT_BORN(fp, device=device, options=options)
+        # the gradient is returned in FP64 and compared as such: its fields keep the rounding that
+        # they have had on every grid
+        for s in (self.forward, self.adjoint):
+            check(lib.cbs_set_transforms(s._h, CBS_TRANSFORMS_FIXED))
         self.RI_inter = None
         self.err_list = []
 
@@ -58,7 +63,7 @@ class BACKWARD_SOLVER_MULTI:
         self.forward._ensure_io()
         if not self.adjoint._io_ready:
             self.adjoint._io_arrays = self.forward._io_arrays
-            from ._lib import check, lib, CBS_MEM_HOST
+            from ._lib import CBS_MEM_HOST
             from .forward_solver import _fptr
             check(lib.cbs_set_io_kernels(self.adjoint._h, *[_fptr(a) for a in self.adjoint._io_arrays],
                                          CBS_MEM_HOST))
@@ -121,7 +126,7 @@ class BACKWARD_SOLVER_MULTI:
         x fastest; complex when cplx): returns the device buffer holding the complex128
         gradient (x fastest) and the misfit."""
         import ctypes as C
-        from ._lib import check, lib, CBS_MEM_DEVICE
+        from ._lib import CBS_MEM_DEVICE
         self._share_io()
         inp = self.forward._inputs(input_field)
         A = inp.shape[3]
@@ -208,7 +213,7 @@ class BACKWARD_SOLVER_MULTI:
         misfit's 2D fields cross to the host, and the RI once at the end."""
         import ctypes as C
         from . import device as dv
-        from ._lib import check, lib, CBS_MEM_DEVICE
+        from ._lib import CBS_MEM_DEVICE
         p = self.parameters
         shape = tuple(RI.shape)
         n = int(np.prod(shape))

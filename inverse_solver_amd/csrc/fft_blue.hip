@@ -1,5 +1,5 @@
-// Bluestein line transforms on compiled convolution lengths (see fft_rt.hpp), for lines of 449 to
-// 648 points; shorter ones run on the matrix cores (fft_dense.hip).
+// Bluestein line transforms on compiled convolution lengths (see fft_rt.hpp): lines of 449 to 648
+// points, and shorter ones under CBS_TRANSFORMS_FIXED (else fft_dense.hip).
 //
 // For a line x of length n with a prime factor above 13,
 //   X_k = conj(c_k) sum_m x_m conj(c_m) c_{k-m},   c_k = exp(i pi k^2 / n),
@@ -377,8 +377,13 @@ __global__ __launch_bounds__(NT) void blue_strided_green(float2* data, Tables tb
 }
 
 // (L, lines per rows block, lines per strided tile, threads): 5-smooth lengths whose
-// two-step plan has both factors <= 36, for the lines that fft_dense.hip does not hold (n > 448)
-#define BLUE_LIST(X) X(1024, 8, 8, 256) X(1152, 8, 8, 256) X(1296, 8, 8, 256)
+// two-step plan has both factors <= 36; those under 1024 are for CBS_TRANSFORMS_FIXED, other
+// handles run lines of up to 448 points on the matrix cores
+#define BLUE_LIST(X)                                                                                           \
+  X(48, 16, 16, 256) X(64, 16, 16, 256) X(80, 16, 16, 256) X(96, 16, 16, 256) X(128, 16, 16, 256)              \
+  X(160, 16, 16, 256) X(192, 16, 16, 256) X(256, 16, 16, 256) X(320, 16, 16, 256) X(384, 16, 16, 256)          \
+  X(512, 16, 16, 256) X(640, 8, 8, 256) X(768, 8, 8, 256) X(1024, 8, 8, 256) X(1152, 8, 8, 256)                \
+  X(1296, 8, 8, 256)
 
 #define BLUE_ENTRY(L, NL, T, NT) \
   {&blue_rows<L, NL, NT>, &blue_strided<L, T, NT>, &blue_rows_update<L, NL, NT>, &blue_strided_green<L, T, NT>, \

@@ -1,7 +1,8 @@
 // Line FFTs of any length, planned at run time (the per-axis form and the 2D
 // convolution-grid transforms of grids whose line lengths have no compiled kernel).
 //
-// Lengths up to 448 run as products with the DFT matrix (fft_dense.hip).  Above, a length n = product of radices from {2, 3, 4, 5, 7, 8, 9, 11, 13, 16} runs as a
+// Lengths up to 448 run as products with the DFT matrix (fft_dense.hip).  Above (and at any length
+// under CBS_TRANSFORMS_FIXED), a length n = product of radices from {2, 3, 4, 5, 7, 8, 9, 11, 13, 16} runs as a
 // mixed-radix Stockham transform (natural order in and out) in LDS, one stage per
 // radix, ping-ponging between two LDS buffers.  Any other n (a prime factor above 13)
 // runs as Bluestein's chirp-z transform: x_n conj(c_n), c_n = exp(i pi n^2 / n), is

@@ -136,7 +136,7 @@ struct RtPlan {
   DevBuf<float2> tw, chirp, bspec;
   const BlueInfo* bi = nullptr;   // Bluestein on a compiled convolution length (else k)
   BlueArgs ba{};
-  int pref = 0;                   // built with prefer_blue
+  int pref = 0;                   // built with prefer_blue (1), dense (2)
   const DenseInfo* di = nullptr;  // products with the DFT matrix (else bi or k)
   DenseArgs da{};
 };
@@ -194,16 +194,17 @@ static void dense_split(int n, DenseArgs& a) {
 // prefer_blue: take Bluestein's transform on a compiled convolution length even when n
 // factors into run-time radices (the per-axis form fuses those transforms with the update
 // and the Green's multiply; run-time stages have no fused form)
-static void build_rt(RtPlan& P, int n, bool prefer_blue = false) {
+// dense: take the matrix-core products where they hold n
+static void build_rt(RtPlan& P, int n, bool dense, bool prefer_blue = false) {
   require(n >= 1, CBS_ERR_ARG, "line length must be >= 1");
   std::vector<int> rs;
   int L = n, blue = 0;
   P.bi = nullptr;
   P.di = nullptr;
-  P.pref = prefer_blue ? 1 : 0;
+  P.pref = (prefer_blue ? 1 : 0) | (dense ? 2 : 0);
   DenseArgs da{};
   dense_split(n, da);
-  P.di = find_dense(n, da.ntask);
+  P.di = dense ? find_dense(n, da.ntask) : nullptr;
   if (P.di) {
     P.k = RtFft{};
     P.k.n = n;
@@ -382,6 +383,25 @@ struct Solver {
   // the convolution grid's x / y transforms (used when io_rows / io_cols are null)
   RtPlan rtp[3], io_rtx, io_rty;
 
+  bool dense = true;              // lengths without a compiled FFT: matrix-core products (cbs_set_transforms)
+
+  void build_io_rt() {            // convolution-grid lengths without a compiled kernel: run-time plans
+    if (!io_rows) build_rt(io_rtx, cx, dense);
+    if (!io_cols) build_rt(io_rty, cy, dense);
+  }
+  void set_transforms(int kind) {
+    if ((kind == CBS_TRANSFORMS_FASTEST) == dense) return;
+    HIP_CHECK(hipStreamSynchronize(stream));
+    dense = kind == CBS_TRANSFORMS_FASTEST;
+    drop_graph();
+    ffp.nx = ffp.ny = 0;
+    if (io.ready) build_io_rt();
+    if (have_potential) {
+      make_plan();
+      build_tables();
+    }
+  }
+
   void rt_rows(const RtPlan& P, float2* data, long long nrows, int inverse) {
     if (P.di) {
       const long long nblk = (nrows + P.di->lines - 1) / P.di->lines;
@@ -553,8 +573,8 @@ struct Solver {
     // 22.0, 22.4, 17.1 and 17.5 to 25.0, 29.3, 26.8 and 22.4 Gvoxel-iter/s)
     const bool fuse = P == 1 && p.form == CBS_FORM_PLAIN;
     for (int j = 0; j < 3; ++j) {
-      const int pref = fuse && j != 1 ? 1 : 0;
-      if (p.rt[j] && (rtp[j].k.n != dims[j] || rtp[j].pref != pref)) build_rt(rtp[j], dims[j], pref);
+      const int pref = (fuse && j != 1 ? 1 : 0) | (dense ? 2 : 0);
+      if (p.rt[j] && (rtp[j].k.n != dims[j] || rtp[j].pref != pref)) build_rt(rtp[j], dims[j], dense, pref & 1);
     }
     p.a = ny;
     p.b = 1;
@@ -1367,8 +1387,7 @@ struct Solver {
             "RI_center other than [0 0]: the reference's crop_field2RI indexes outside the field grid");
     io_rows = find_fft_rows(cx);
     io_cols = find_fft_strided(cy, 0);
-    if (!io_rows) build_rt(io_rtx, cx);    // lengths without a compiled kernel: run-time plans
-    if (!io_cols) build_rt(io_rty, cy);
+    build_io_rt();
     const size_t n = (size_t)cx * cy * rz;
     const hipMemcpyKind kind = mem == CBS_MEM_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
     io_refocus_k.ensure(n);
@@ -1487,8 +1506,8 @@ struct Solver {
     if (ffp.nx != fx || ffp.ny != fy) {
       ffp.rw = find_fft_rows(fx);
       ffp.st = find_fft_strided(fy, 0);
-      if (!ffp.rw) build_rt(ffp.rtx, fx);
-      if (!ffp.st) build_rt(ffp.rty, fy);
+      if (!ffp.rw) build_rt(ffp.rtx, fx, dense);
+      if (!ffp.st) build_rt(ffp.rty, fy, dense);
       ffp.twx.upload(twiddles(fx));
       ffp.twy.upload(twiddles(fy));
       ffp.nx = fx;
@@ -2509,6 +2528,15 @@ int cbs_set_convergence(cbs_handle h, double tol) {
     HIP_CHECK(hipStreamSynchronize(s->stream));
     s->conv_tol = tol;
     s->drop_graph();
+  });
+}
+
+int cbs_set_transforms(cbs_handle h, int kind) {
+  return guarded([&] {
+    Solver* s = lookup(h);
+    require(kind == CBS_TRANSFORMS_FASTEST || kind == CBS_TRANSFORMS_FIXED, CBS_ERR_ARG, "unknown kind of transforms");
+    DeviceGuard dg(s->device);
+    s->set_transforms(kind);
   });
 }
 
