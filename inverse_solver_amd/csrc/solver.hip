@@ -512,16 +512,26 @@ struct Solver {
       const int npr = list_pass_real(&prs);
       const PassKInfo* pks = nullptr;
       const int npk = list_pass_kspace(&pks);
-      // default preference: the largest a whose LDS tile keeps two blocks per CU
-      // (<= 80 KiB), then the widest x tile, then 256 threads; cbs_autotune
-      // replaces this choice by measurement.
-      // (measured on MI355X at 160^3 x 49 rhs: 512-thread blocks beat 256 for
-      // tiles of 40 KiB and more)
+      // default preference; cbs_autotune replaces it by measurement.
+      // Scalar runs: the largest b <= 4 whose real-space tile still holds 2048 points and whose
+      // k-space tile can be 16 wide, else b = 2; then a 32-wide x tile for b <= 2, a 16-wide one above
+      // (64 KB and less).  With 20-iteration solves, ms, of 1, 12 and 49 rhs at 96^3: b = 1 (largest a)
+      // 0.66, 2.85, 10.42; b = 2, 32-wide 0.55, 2.65, 9.71; b = 4, 16-wide 0.55, 2.54, 9.30; of 1, 4
+      // and 24 rhs at 128^2 x 135 (no 16-wide tile with b = 4): b = 2, 16-wide 0.93, 2.49, 12.11, 32-wide
+      // 0.89, 2.44, 12.15; b = 4, 8-wide 0.87, 2.49, 13.62; of 1 and 49 rhs at 40^3: b = 1 0.28, 1.01; b = 2 0.25, 0.97.  160^3 and 192^2 x 128 have b = 4 either way.
+      // Vector runs: the largest a whose tile keeps two blocks per CU (<= 80 KiB), then the
+      // narrowest x tile of 16 and more.
+      // Threads: 512 for tiles of 40 KiB and more, else 256 (160^3 x 49 rhs).
       auto score_r = [&](const PassRInfo& r) {
-        return (r.lds <= 81920 ? 1000000 : 0) + r.a * 10 + ((r.nt == 512) == (r.lds >= 40960) ? 1 : 0);
+        const int b = ny / r.a;
+        bool wide = false;   // a 16-wide x tile with this b
+        for (int j = 0; j < npk; ++j) wide = wide || (fused_ok_k(pks[j], b) && pks[j].t >= 16);
+        const int pref = P > 1 ? r.a * 10 : wide && b <= 4 && r.a * r.nx >= 2048 ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
+        return (r.lds <= 81920 ? 1000000 : 0) + pref + ((r.nt == 512) == (r.lds >= 40960) ? 1 : 0);
       };
       auto score_k = [&](const PassKInfo& q) {
-        return (q.lds <= 81920 ? 1000 : 0) + (q.t >= 16 ? 100 : 0) - q.t + ((q.nt == 512) == (q.lds >= 40960) ? 1 : 0);
+        return (q.lds <= 81920 ? 1000 : 0) + (q.t >= 16 ? 100 : 0) + (P == 1 && q.b <= 2 ? q.t : -q.t) +
+               ((q.nt == 512) == (q.lds >= 40960) ? 1 : 0);
       };
       long best = -1;
       for (int i = 0; i < npr; ++i) {
