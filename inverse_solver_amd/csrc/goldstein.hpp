@@ -137,23 +137,19 @@ __host__ __device__ inline void nearest(const unsigned char* state, const int32_
 
 // ---- host part: listing and the sequential branch search
 
-// goldstein_branch_cut.m:7-38: list, order and index the residues of a dipole-free map.
+// goldstein_branch_cut.m:7-38: list, order and index the residues of a dipole-free map: flat
+// indices in ascending order and their values.
 struct GsList {
   int n = 0;
   std::vector<int32_t> rows;                  // 6 per residue, see goldstein.hpp
   std::vector<int32_t> square, zstart, table;
 };
 
-inline GsList gs_list(const std::vector<float>& res, int m1, int m2, int n3) {
+inline GsList gs_list(const std::vector<long long>& idx, const std::vector<float>& val, int m1, int m2, int n3) {
   GsList L;
   const long long plane = (long long)m1 * m2;
-  std::vector<long long> idx;
   std::vector<int> count(n3, 0);
-  for (long long i = 0; i < (long long)res.size(); ++i)
-    if (res[i] != 0.0f) {
-      idx.push_back(i);
-      ++count[(int)(i / plane)];
-    }
+  for (long long i : idx) ++count[(int)(i / plane)];
   L.square.resize(n3);
   L.zstart.resize(n3);
   int size = 0;
@@ -172,7 +168,7 @@ inline GsList gs_list(const std::vector<float>& res, int m1, int m2, int n3) {
     const int c = d1 / case_side(m1, sq) + (d2 / case_side(m2, sq)) * sq;
     int32_t* r = &rows[6 * (size_t)k];
     r[kIdx] = (int32_t)i;
-    r[kVal] = (int32_t)std::lrint(res[i]);
+    r[kVal] = (int32_t)std::lrint(val[k]);
     r[kCase] = c;
     r[kX] = d1;
     r[kY] = d2;
