@@ -139,9 +139,11 @@ void pass_real(PassRArgs args) {
   };
   float2* __restrict__ F = args.st.field + roff + zoff;
   float2* __restrict__ f = args.st.fstate + roff + zoff;
-  // small tiles (few blocks, e.g. a single rhs): the pointwise operands are requested with
-  // the tile, so their latency overlaps the inverse transforms instead of following them
-  constexpr bool PF = L <= 5;
+  // few pairs a thread: the pointwise operands are requested with the tile, so their latency
+  // overlaps the inverse transforms instead of following them.  They take 12 registers a pair: from
+  // four pairs on the occupancy they cost weighs more (96 x 24 tiles on 256 threads, 4 rhs of 96^3:
+  // 53.2 us an iteration with five pairs held, 45.9 without).
+  constexpr bool PF = L <= 3;
   constexpr int LP = PF ? L : 1;
   float4 pv[LP], px[LP], pF[LP];
   if constexpr (PF) {

@@ -124,6 +124,8 @@ struct Plan {
   int a = 0, b = 0, t = 0;
   const PassRInfo* pr = nullptr;
   const PassKInfo* pk = nullptr;
+  const PassRInfo* pr_few = nullptr;   // fused form: the passes of launches with few blocks (run_fused)
+  const PassKInfo* pk_few = nullptr;
   const RowsInfo* rw = nullptr;
   const StridedInfo* sy = nullptr;
   const StridedInfo* sz = nullptr;
@@ -514,24 +516,30 @@ struct Solver {
       const int npk = list_pass_kspace(&pks);
       // default preference; cbs_autotune replaces it by measurement.
       // Scalar runs: the largest b <= 4 whose real-space tile still holds 2048 points and whose
-      // k-space tile can be 16 wide, else b = 2; then a 32-wide x tile for b <= 2, a 16-wide one above
-      // (64 KB and less).  With 20-iteration solves, ms, of 1, 12 and 49 rhs at 96^3: b = 1 (largest a)
-      // 0.66, 2.85, 10.42; b = 2, 32-wide 0.55, 2.65, 9.71; b = 4, 16-wide 0.55, 2.54, 9.30; of 1, 4
-      // and 24 rhs at 128^2 x 135 (no 16-wide tile with b = 4): b = 2, 16-wide 0.93, 2.49, 12.11, 32-wide
-      // 0.89, 2.44, 12.15; b = 4, 8-wide 0.87, 2.49, 13.62; of 1 and 49 rhs at 40^3: b = 1 0.28, 1.01; b = 2 0.25, 0.97.  160^3 and 192^2 x 128 have b = 4 either way.
-      // Vector runs: the largest a whose tile keeps two blocks per CU (<= 80 KiB), then the
-      // narrowest x tile of 16 and more.
-      // Threads: 512 for tiles of 40 KiB and more, else 256 (160^3 x 49 rhs).
+      // k-space tile can be 16 wide, else b = 2; then an x tile of 8 and more that divides nx, 32 wide
+      // for b <= 2 and 16 wide above.  Iterations, us, of 1, 4 and 24 rhs at 96^3: b = 1 (largest
+      // a) 32, 50, 245; b = 2 24.2, 44.3, 229; b = 4 23.9, 44.7, 227; at 128^2 x 135: b = 2 42.6, 119, 590;
+      // b = 4 36.4, 106, 555; of 1 and 16 rhs at 40^3 (8-wide tiles, 16-wide ones run past the row):
+      // b = 1 13.1, 27.4; b = 2 10.3, 23.1; of 4 rhs at 288^2 x 160, b = 9: 8-wide (92 KB, one block a
+      // CU) 741, 4-wide (32-byte rows) 808.  160^3 and 192^2 x 128 have b = 4 either way.
+      // Vector runs, and runs whose transforms keep their rounding (cbs_set_transforms): the largest a
+      // whose tile keeps two blocks per CU (<= 80 KiB); vector runs then the narrowest x tile of 16 and more.
+      // Threads: real space 512 for tiles of 32 KiB and more (128 x 32, 24 rhs: 14.8 against
+      // 15.1 us on 256), else 256; k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 26.1 against 27.4
+      // on 512 and 32.3 on 1024), 512 from 40 KiB (96^3 x 24: 2.8; 768 threads 3.1, 256 3.1).
+      const bool keep = P > 1 || !dense;
       auto score_r = [&](const PassRInfo& r) {
         const int b = ny / r.a;
         bool wide = false;   // a 16-wide x tile with this b
         for (int j = 0; j < npk; ++j) wide = wide || (fused_ok_k(pks[j], b) && pks[j].t >= 16);
-        const int pref = P > 1 ? r.a * 10 : wide && b <= 4 && r.a * r.nx >= 2048 ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
-        return (r.lds <= 81920 ? 1000000 : 0) + pref + ((r.nt == 512) == (r.lds >= 40960) ? 1 : 0);
+        const int pref = keep ? r.a * 10 : wide && b <= 4 && r.a * r.nx >= 2048 ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
+        return (r.lds <= 81920 ? 1000000 : 0) + pref + (r.nt == (r.lds >= 32768 ? 512 : 256) ? 1 : 0);
       };
       auto score_k = [&](const PassKInfo& q) {
-        return (q.lds <= 81920 ? 1000 : 0) + (q.t >= 16 ? 100 : 0) + (P == 1 && q.b <= 2 ? q.t : -q.t) +
-               ((q.nt == 512) == (q.lds >= 40960) ? 1 : 0);
+        const int want = P > 1 ? 512 : q.lds >= 64000 ? 768 : 512;
+        const int nt = q.lds < 40960 ? (q.nt < 512 ? 1 : 0) : q.nt == want ? 2 : q.nt == 512 ? 1 : 0;
+        return 4 * ((P == 1 && q.t >= 8 ? 2000 : 0) + (q.lds <= 81920 ? 1000 : 0) +
+                    (P == 1 && nx % q.t == 0 ? 200 : 0) + (q.t >= 16 ? 100 : 0) + (P == 1 && q.b <= 2 ? q.t : -q.t)) + nt;
       };
       long best = -1;
       for (int i = 0; i < npr; ++i) {
@@ -545,7 +553,7 @@ struct Solver {
           if (!k || score_k(q) > score_k(*k)) k = &q;
         }
         if (!k) continue;
-        const long sc = (long)score_r(r) * 10000 + score_k(*k);
+        const long sc = (long)score_r(r) * 100000 + score_k(*k);
         if (sc > best) {
           best = sc;
           p.pr = &r;
@@ -556,6 +564,17 @@ struct Solver {
         p.a = p.pr->a;
         p.b = ny / p.a;
         p.t = p.pk->t;
+        // Launches of few blocks (run_fused): the real-space variant with the most threads, the narrowest
+        // k-space tile of 4 and more.  One rhs of 96^3: 27.5 -> 23.9 us an iteration (576 threads 2.4 us
+        // of it), of 40^3 10.7 -> 10.3; at 4 rhs the wide forms are as fast or faster.
+        p.pr_few = p.pr;
+        p.pk_few = p.pk;
+        if (opt.threads_real == 0)
+          for (int i = 0; i < npr; ++i)
+            if (fused_ok_r(prs[i]) && prs[i].a == p.a && prs[i].nt > p.pr_few->nt) p.pr_few = &prs[i];
+        if (P == 1 && opt.threads_kspace == 0 && opt.tile_t == 0)
+          for (int j = 0; j < npk; ++j)
+            if (fused_ok_k(pks[j], p.b) && pks[j].t >= 4 && pks[j].t < p.pk_few->t) p.pk_few = &pks[j];
         plan = p;
         return;
       }
@@ -838,9 +857,11 @@ struct Solver {
 
   // fused schedule for one batch already seeded in fstate
   void run_fused(int nb, int M) {
-    const PassRInfo* pr = plan.pr;
-    const PassKInfo* pk = plan.pk;
     const int nv = nb * P;                 // component slots: the real-space pass treats each as an rhs
+    // few blocks: two real-space blocks a CU or less, fewer k-space blocks than CUs (256)
+    const PassRInfo* pr = plan.pr_few && (long long)nv * plan.b * nz <= 512 ? plan.pr_few : plan.pr;
+    const PassKInfo* pk =
+        plan.pk_few && (long long)nb * plan.a * ((nx + plan.t - 1) / plan.t) < 256 ? plan.pk_few : plan.pk;
     const Consts c = consts(nv);
     const Consts ck = consts(nb);
     const Tables tb = tabs.view();
@@ -1739,14 +1760,22 @@ struct Solver {
     const cbs_options saved = opt;
     opt.split_a = opt.tile_t = opt.threads_real = opt.threads_kspace = 0;
     opt.form = CBS_FORM_FUSED;
+    // transforms that keep their rounding keep the planner's split of y, which sets it
+    if (!dense) make_plan();
+    const int keep_a = !dense && plan.form == CBS_FORM_FUSED ? plan.a : 0;
     std::vector<std::pair<const PassRInfo*, const PassKInfo*>> cands;
     for (int i = 0; i < npr; ++i) {
       if (!fused_ok_r(prs[i])) continue;
+      if (keep_a > 0 && prs[i].a != keep_a) continue;
       for (int j = 0; j < npk; ++j)
         if (fused_ok_k(pks[j], ny / prs[i].a)) cands.emplace_back(&prs[i], &pks[j]);
     }
     if (cands.empty()) {
       opt = saved;
+      if (!dense) {
+        make_plan();
+        build_tables();
+      }
       throw CbsError(CBS_ERR_UNSUPPORTED, "no fused kernel plan to tune for grid " + shape_str());
     }
     const int nb = batch_width(n_rhs);
