@@ -49,7 +49,7 @@ struct PassRArgs {
 constexpr int pass_real_min_waves(int nx, int a, int nt) { return nx == 160 && a == 40 && nt == 512 ? 6 : 1; }
 
 //
-// VR = 1 (fused form, real RI): V is read as its real part from st.Vr, 4 bytes a voxel,
+// VR = 1 (real RI): V is read as its real part from st.Vr, 4 bytes a voxel,
 // with the imaginary part -eps that V holds at every voxel for a real RI.
 template <int NX, int A, int NT, int ROWS, int STEADY, int VR>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(pass_real_min_waves(NX, A, NT))))
@@ -669,7 +669,8 @@ void pass_kspace_seq3(PassKArgs args) {
 // transform, fwd = FWD_NONE the forward one; a slot the convergence test has stopped
 // leaves Field, f and the spectrum alone after the flush of a deferred increment.  Every
 // global operand of a thread's elements is requested before the first transform.
-template <int N, int NL, int NT>
+// VR = 1 (real RI): the potential is read as its real part from st.Vr, as in pass_real.
+template <int N, int NL, int NT, int VR>
 __global__ __launch_bounds__(NT) void line_rows_update(StateArgs st, Tables tb, Consts c, const float2* tw, int upd,
                                                        int fwd, int jj_inv, int jj_fwd, ConvArgs cv) {
   constexpr int PR = row_pitch(N);
@@ -684,6 +685,7 @@ __global__ __launch_bounds__(NT) void line_rows_update(StateArgs st, Tables tb, 
   float2* __restrict__ F = st.field + ro;
   float2* __restrict__ f = st.fstate + ro;
   const float2* __restrict__ V = st.V + (long long)r0 * N;
+  const float* __restrict__ Vr = VR ? st.Vr + (long long)r0 * N : nullptr;
   if (cv.norms && jj_inv > 0) {
     const int rr = slot / cv.P;
     if (conv_stopped(cv, jj_inv - 1, rr)) {
@@ -702,7 +704,8 @@ __global__ __launch_bounds__(NT) void line_rows_update(StateArgs st, Tables tb, 
     xq[k] = vv[k] = xo[k] = Fo[k] = make_float2(0.f, 0.f);
     if (i < nr * N) {
       if (rq) xq[k] = spec[i];
-      vv[k] = V[i];
+      if constexpr (VR) vv[k] = make_float2(Vr[i], -c.eps);
+      else vv[k] = V[i];
       if (rf) xo[k] = f[i];
       if (rF) Fo[k] = F[i];
     }

@@ -181,14 +181,35 @@ constexpr int kRW = kL * 64 / kNT;
 constexpr int kPR = kL + 1;        // lanes walking a row spread over the banks
 constexpr int tables_k(int n, int nt) { return (2 * n + nt - 1) / nt; }
 
-template <int EC>
-__device__ __forceinline__ void load_rows(const float2* __restrict__ base, int n, int nr, int w, int lane,
-                                          float2 (&v)[kRW * EC]) {
+template <int EC, class T>
+__device__ __forceinline__ void load_rows(const T* __restrict__ base, int n, int nr, int w, int lane,
+                                          T (&v)[kRW * EC]) {
 #pragma unroll
   for (int k = 0; k < kRW; ++k) {
-    const float2* __restrict__ row = base + min(w * kRW + k, nr - 1) * n;
+    const T* __restrict__ row = base + min(w * kRW + k, nr - 1) * n;
 #pragma unroll
-    for (int ch = 0; ch < EC; ++ch) v[k * EC + ch] = *byte_at<const float2>(row, 8u * (unsigned)min(lane + 64 * ch, n - 1));
+    for (int ch = 0; ch < EC; ++ch)
+      v[k * EC + ch] = *byte_at<const T>(row, (unsigned)sizeof(T) * (unsigned)min(lane + 64 * ch, n - 1));
+  }
+}
+// The potential of the rows: re and im of every element, the imaginary part in memory only where st.Vr is null.
+template <int EC>
+__device__ __forceinline__ void load_potential(const StateArgs& st, const Consts& c, int r0, int n, int nr, int w, int lane,
+                                               float2 (&v)[kRW * EC]) {
+  const bool real = st.Vr != nullptr;
+  const unsigned sz = real ? 4u : 8u;
+  const char* __restrict__ base = (real ? reinterpret_cast<const char*>(st.Vr) : reinterpret_cast<const char*>(st.V)) +
+                                  (long long)r0 * n * sz;
+#pragma unroll
+  for (int k = 0; k < kRW; ++k) {
+    const char* __restrict__ row = base + (long long)(min(w * kRW + k, nr - 1) * n) * sz;
+#pragma unroll
+    for (int ch = 0; ch < EC; ++ch) {
+      const unsigned o = sz * (unsigned)min(lane + 64 * ch, n - 1);
+      v[k * EC + ch].x = *byte_at<const float>(row, o);
+      v[k * EC + ch].y = -c.eps;
+      if (!real) v[k * EC + ch].y = *byte_at<const float>(row, o + 4u);
+    }
   }
 }
 template <int EC>
@@ -259,7 +280,6 @@ void dense_rows_update(StateArgs st, Tables tb, Consts c, DenseArgs p, int upd_,
   float2* __restrict__ spec = st.spec + ro;
   float2* __restrict__ F = st.field + ro;
   float2* __restrict__ f = st.fstate + ro;
-  const float2* __restrict__ V = st.V + (long long)r0 * n;
   if (cv.norms && jj_inv > 0) {
     const int rr = slot / cv.P;
     if (conv_stopped(cv, jj_inv - 1, rr)) {
@@ -294,7 +314,7 @@ void dense_rows_update(StateArgs st, Tables tb, Consts c, DenseArgs p, int upd_,
   }
   tabs.store(s_tw, tid);
   if (rq) put_rows<EC>(lds, n, w, lane, xq);
-  load_rows<EC>(V, n, nr, w, lane, vv);
+  load_potential<EC>(st, c, r0, n, nr, w, lane, vv);
   if (rf) load_rows<EC>(f, n, nr, w, lane, xo);
   if (rF) load_rows<EC>(F, n, nr, w, lane, Fo);
   lds_barrier();

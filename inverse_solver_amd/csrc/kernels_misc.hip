@@ -159,7 +159,7 @@ __global__ void tile_rows(const float2* __restrict__ V, float2* __restrict__ Vt,
   }
 }
 
-// Re V in the state arrays' row order (V natural -> Vr, c.tiled = 1), for a potential
+// Re V in the state arrays' row order (V natural -> Vr), for a potential
 // whose imaginary part is -eps everywhere (a real RI).
 __global__ void tile_rows_real(const float2* __restrict__ V, float* __restrict__ Vr, Consts c) {
   GRID_STRIDE(i, c.nvox) {

@@ -43,7 +43,7 @@ using RowsFn = void (*)(float2*, long long, const float2*, int);
 using StridedFn = void (*)(float2*, int, long long, long long, int, const float2*, int, int, long long);
 
 // fn takes every update kind; fn_steady only UPD_DEFER / UPD_PAIR with FWD_GAMMA
-// fn_vr, fn_steady_vr: the same passes reading a real potential (st.Vr; fused form only)
+// fn_vr, fn_steady_vr: the same passes reading a real potential (st.Vr)
 struct PassRInfo { PassRFn fn, fn_steady, fn_vr, fn_steady_vr; int nx, a, nt, lds, rows; };
 struct PassKInfo { PassKFn fn; int b, nz, t, nt, lds, pole; };
 struct RowsInfo { RowsFn fn; int n, rows, nt; };
@@ -57,7 +57,7 @@ const StridedInfo* find_fft_strided(int n, int t);
 // x inverse + pointwise update + x forward, and z forward + Green's multiply + z inverse
 using RowsUpdateFn = void (*)(StateArgs, Tables, Consts, const float2*, int, int, int, int, ConvArgs);
 using StridedGreenFn = void (*)(float2*, Tables, Consts, const float2*, const uint8_t*, int, ConvArgs);
-struct RowsUpdateInfo { RowsUpdateFn fn; int n, rows, nt; };
+struct RowsUpdateInfo { RowsUpdateFn fn, fn_vr; int n, rows, nt; };   // fn_vr: real potential (st.Vr)
 struct StridedGreenInfo { StridedGreenFn fn; int n, t, nt; };
 const RowsUpdateInfo* find_rows_update(int n);
 const StridedGreenInfo* find_strided_green(int n);

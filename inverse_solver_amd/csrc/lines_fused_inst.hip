@@ -17,7 +17,7 @@ namespace cbs {
 constexpr int fused_rows(int n) { return n <= 64 ? 16 : (n <= 256 ? 8 : (n <= 576 ? 4 : 2)); }
 constexpr int fused_t(int n) { return n <= 576 ? 16 : 8; }
 
-#define RU_ENTRY(N) {&line_rows_update<N, fused_rows(N), 256>, N, fused_rows(N), 256},
+#define RU_ENTRY(N) {&line_rows_update<N, fused_rows(N), 256, 0>, &line_rows_update<N, fused_rows(N), 256, 1>, N, fused_rows(N), 256},
 #define SG_ENTRY(N) {&line_strided_green<N, fused_t(N), 256>, N, fused_t(N), 256},
 
 static const RowsUpdateInfo kRU[] = {FUSED_LIST(RU_ENTRY)};

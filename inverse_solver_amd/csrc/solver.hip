@@ -326,8 +326,8 @@ struct Solver {
   bool have_potential = false;
   cbs_potential_params prm{};
   DevBuf<float2> V;
-  // the fused form's copy of V in the state arrays' tile row order (state_row), made when
-  // the potential or the plan changes, never inside a solve: Vt, or for a real RI (V's
+  // copies of V in the state arrays' row order (state_row: the fused form's tiles), made when
+  // the potential or the plan changes, never inside a solve: the fused form's Vt, or for a real RI (V's
   // imaginary part -eps everywhere, as potential_fill forms it) only its real part, Vr
   DevBuf<float2> Vt;
   DevBuf<float> Vr;
@@ -824,9 +824,8 @@ struct Solver {
   StateArgs state_args(int nb) {
     (void)nb;
     StateArgs s;
-    const bool fused = plan.form == CBS_FORM_FUSED;
-    s.V = fused && !v_real ? Vt.p : V.p;
-    s.Vr = fused && v_real ? Vr.p : nullptr;
+    s.V = plan.form == CBS_FORM_FUSED && !v_real ? Vt.p : V.p;
+    s.Vr = has_vr() ? Vr.p : nullptr;
     s.field = ws.field; s.fstate = ws.fstate; s.spec = ws.spec; s.parity = ws.parity;
     s.rhs_stride = nvox;
     s.norms = nullptr;
@@ -879,7 +878,6 @@ struct Solver {
       const bool steady = (upd == UPD_DEFER || upd == UPD_PAIR) && fwd == FWD_GAMMA;
       const bool vr = args.st.Vr != nullptr;   // real potential: its 4-byte form
       const PassRFn fn = steady ? (vr ? pr->fn_steady_vr : pr->fn_steady) : (vr ? pr->fn_vr : pr->fn);
-      require(fn != nullptr, CBS_ERR_UNSUPPORTED, "no real-potential form of the real-space pass");
       timed(0, [&] { hipLaunchKernelGGL(fn, grid, dim3(pr->nt), 0, stream, args); });
     };
     auto pass_k = [&](int jj) {
@@ -922,12 +920,13 @@ struct Solver {
       args.st.norms = norm_row(jj_inv, nv);
       if (conv_tol > 0.0 && upd == UPD_VQ_ADD) args.st.fref = ws.fref;
       args.upd = upd; args.fwd = fwd; args.jj_inv = jj_inv; args.jj_fwd = jj_fwd;
-      args.order = 0;
+      args.order = 0;   // rhs that share a row of the potential together (storage order: 2 % longer at 576^2 x 320 x 4)
       args.nt = stream_hint(nv);
       args.cv = cv;
       const dim3 grid((unsigned)((long long)nv * plan.b * nz));
       const bool steady = (upd == UPD_DEFER || upd == UPD_PAIR) && fwd == FWD_GAMMA;
-      const PassRFn fn = steady ? pr->fn_steady : pr->fn;
+      const bool vr = args.st.Vr != nullptr;
+      const PassRFn fn = steady ? (vr ? pr->fn_steady_vr : pr->fn_steady) : (vr ? pr->fn_vr : pr->fn);
       timed(0, [&] { hipLaunchKernelGGL(fn, grid, dim3(pr->nt), 0, stream, args); });
     };
     auto pass_k = [&](int jj) {
@@ -1046,7 +1045,7 @@ struct Solver {
         timed(2, [&] { hipLaunchKernelGGL(bx->rows_update, g, dim3(bx->nt), 0, stream, s, tb, c, rtp[0].ba, upd, fwd,
                                           jj_inv, jj_fwd, cv); });
       else
-        timed(2, [&] { hipLaunchKernelGGL(cx->fn, g, dim3(cx->nt), 0, stream, s, tb, c, tabs.tw_x.p, upd, fwd,
+        timed(2, [&] { hipLaunchKernelGGL(s.Vr ? cx->fn_vr : cx->fn, g, dim3(cx->nt), 0, stream, s, tb, c, tabs.tw_x.p, upd, fwd,
                                           jj_inv, jj_fwd, cv); });
     };
     auto zpass = [&](int jj) {   // z forward, Green's multiply, z inverse
@@ -1119,7 +1118,8 @@ struct Solver {
     uint64_t b = 3ull * nv * nvox * sizeof(float2);   // field, fstate, spec
     b += 2ull * nv * nri * sizeof(float2);             // staging for host I/O
     b += (uint64_t)nvox * sizeof(float2);   // V
-    if (plan.form == CBS_FORM_FUSED) b += (uint64_t)nvox * (v_real ? sizeof(float) : sizeof(float2));   // its tile-order copy
+    if (has_vr()) b += (uint64_t)nvox * sizeof(float);
+    else if (plan.form == CBS_FORM_FUSED) b += (uint64_t)nvox * sizeof(float2);   // its tile-order copy
     b += io.footprint(nv, cx, cy, rz) + (io.ready ? (unsigned long long)nv * nri * 16ull : 0ull);
     return b;
   }
@@ -2054,10 +2054,17 @@ struct Solver {
     finish_potential();
   }
 
-  // Vt for the fused plan (its a and b) from the current V
+  // a real RI's potential is read as Vr by the real-space passes and the x transforms fused with the update:
+  // 4 bytes a voxel less of 40 or 56 (576^2 x 320 x 4 rhs 527.8 -> 523.1 ms, 263 x 238 x 129 x 6 40.8 -> 40.0)
+  bool has_vr() const {
+    return v_real && (plan.form == CBS_FORM_FUSED || plan.form == CBS_FORM_ROWS ||
+                      (plan.form == CBS_FORM_PLAIN && P == 1));
+  }
+  // Vt (the fused plan's a and b) or Vr from the current V
   void sync_vtile() {
-    if (plan.form != CBS_FORM_FUSED || !V.p) return;
-    const std::vector<long long> key = {v_version, (long long)plan.a, (long long)plan.b, nvox, (long long)v_real};
+    if ((plan.form != CBS_FORM_FUSED && !has_vr()) || !V.p) return;
+    const std::vector<long long> key = {v_version, (long long)plan.form, (long long)plan.a, (long long)plan.b, nvox,
+                                        (long long)v_real};
     if (key == vt_key) return;
     if (v_real) {
       Vr.ensure((size_t)nvox);
