@@ -1918,7 +1918,7 @@ struct Solver {
     const size_t esz = cplx ? sizeof(float2) : sizeof(float);
     const long long nf = cplx ? 2 * n : n;   // floats per volume
     tv_y.ensure((size_t)n);
-    tv_P.ensure((size_t)(9 * n));   // P_{k-1}, P_k and P_{k+1}
+    tv_P.ensure((size_t)(12 * n));   // P_{k-1}, P_k, P_{k+1} and P_{k+2}
     const void* din = in;
     if (mem == CBS_MEM_HOST) {
       tv_in.ensure((size_t)n);
@@ -1930,26 +1930,51 @@ struct Solver {
     a.lam = (float)lam; a.vmin = (float)vmin; a.vmax = (float)vmax;
     a.vimag_max = (vimag_max > 0) ? (float)vimag_max : 0.f;   // NaN or <= 0: no cap (the reference tests > 0)
     a.non_neg = non_neg; a.dirichlet = dirichlet;
-    float* Pk[3];
-    for (int k = 0; k < 3; ++k) Pk[k] = reinterpret_cast<float*>(tv_P.p) + (size_t)k * 3 * nf;
+    float* Pk[4];
+    for (int k = 0; k < 4; ++k) Pk[k] = reinterpret_cast<float*>(tv_P.p) + (size_t)k * 3 * nf;
     float* Y = reinterpret_cast<float*>(tv_y.p);
     if (inner == 0) hipLaunchKernelGGL(tv_zero, dim3(grid_for(3 * nf)), dim3(256), 0, stream, Pk[0], 3 * nf);
     const unsigned g = grid_for(n);
-    int cur = 0;                // P_k in Pk[cur], P_{k-1} in the one before it
+    int cur = 0, prv = 0;       // P_k in Pk[cur], P_{k-1} in Pk[prv]
     double t = 1.0;
-    float theta = 0.f;          // the momentum between P_k and P_{k-1}
-    for (uint32_t it = 0; it < inner; ++it) {
+    // the momentum between the two newest iterates after each iteration
+    auto momentum = [&t] {
       const double tn = (1.0 + std::sqrt(1.0 + 4.0 * t * t)) / 2.0;
-      // theta is 0 after the first iteration: P_1 stands in for the P_0 = 0 that no buffer holds
-      const int nxt = (cur + 1) % 3, prv = it == 1 ? cur : (cur + 2) % 3;
-      if (cplx)
-        tv_inner_complex(stream, (const float2*)din, (const float2*)Pk[cur], (const float2*)Pk[prv], (float2*)Pk[nxt],
-                         a, theta, it == 0);
-      else
-        tv_inner_real(stream, (const float*)din, Pk[cur], Pk[prv], Pk[nxt], a, theta, it == 0);
-      theta = (float)((t - 1.0) / tn);
+      const float theta = (float)((t - 1.0) / tn);
       t = tn;
-      cur = nxt;
+      return theta;
+    };
+    float theta = 0.f;
+    // the first iteration reads no iterate (P_0 = 0); theta is 0 after it, and P_1 stands in for P_0.  The
+    // others go two to a launch where that is faster
+    const TvTiles tiles = tv_tiles(a, cplx);
+    for (uint32_t it = 0; it < inner;) {
+      // the two buffers that hold neither P_k nor P_{k-1}
+      int nxt[2], m = 0;
+      for (int k = 0; k < 4 && m < 2; ++k)
+        if (k != cur && k != prv) nxt[m++] = k;
+      if (it > 0 && it + 1 < inner && tiles.gz > 0) {
+        const float theta1 = momentum();
+        if (cplx)
+          tv_inner2_complex(stream, (const float2*)din, (const float2*)Pk[cur], (const float2*)Pk[prv],
+                            (float2*)Pk[nxt[0]], (float2*)Pk[nxt[1]], a, tiles, theta, theta1);
+        else
+          tv_inner2_real(stream, (const float*)din, Pk[cur], Pk[prv], Pk[nxt[0]], Pk[nxt[1]], a, tiles, theta, theta1);
+        theta = momentum();
+        prv = nxt[0];
+        cur = nxt[1];
+        it += 2;
+        continue;
+      }
+      if (cplx)
+        tv_inner_complex(stream, (const float2*)din, (const float2*)Pk[cur], (const float2*)Pk[prv],
+                         (float2*)Pk[nxt[0]], a, theta, it == 0);
+      else
+        tv_inner_real(stream, (const float*)din, Pk[cur], Pk[prv], Pk[nxt[0]], a, theta, it == 0);
+      theta = momentum();
+      prv = it == 0 ? nxt[0] : cur;
+      cur = nxt[0];
+      ++it;
     }
     void* dst = mem == CBS_MEM_HOST ? (void*)Y : out;
     if (cplx)

@@ -176,6 +176,153 @@ __global__ __launch_bounds__(kTvX * kTvY) void tv_inner(const T* __restrict__ in
   }
 }
 
+// Two inner iterations in one launch: reads P_k, P_{k-1} and in, writes P1 = P_{k+1} and P2 = P_{k+2},
+// 13 values a voxel where two launches of tv_inner move 20, with one start and drain of the chip for two.
+//
+// P_{k+2} of a voxel needs P_{k+1} of its neighbours and that their y, so a block of TX x TY threads, a
+// thread a column, holds two more columns on each side than it writes and walks up z through its planes,
+// two planes more below and two steps more above.  In the step that takes plane a, the first iteration's y
+// of plane a and the second one's y of plane b = a - 2 share the LDS passes and their two barriers; P1 of
+// plane a - 1 and P2 of plane b - 1 leave it.  Every value is the expression of tv_inner.
+// theta: the momentum between P_k and P_{k-1}; theta1: between P1 and P_k.
+// A step is bound by the latency of its barriers and of the operands, requested D planes ahead: two for real
+// input (78 registers, two blocks a CU), one for complex (105, one block a CU; two ahead: 18.6 for 18.0 us).
+// An iteration, us: real 96 x 96 x 97 10.4 (tv_inner) -> 8.6, 200 x 190 x 110 35.5 -> 24.6; complex
+// 161 x 161 x 61 26.7 -> 18.0, 200 x 190 x 110 85.5 -> 55.7, 100 x 110 x 100 20.9 -> 14.6.  With 1024 and
+// 512 threads the 161 x 161 x 61 and 200 x 190 x 110 complex take 19.9 and 19.7, 59.5 and 61.9.
+constexpr int kTvT2 = 768;
+template <class T, class Off>
+__global__ __launch_bounds__(kTvT2) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 3)))
+void tv_inner2(const T* __restrict__ in, const T* __restrict__ Pc,
+                                                   const T* __restrict__ Pp, T* __restrict__ P1, T* __restrict__ P2,
+                                                   TvArgs a, TvTiles g, float theta, float theta1) {
+  __shared__ T sx[kTvT2], sz[kTvT2], sy[kTvT2];   // R_x, R_y and y of the first iteration, plane a
+  __shared__ T tx1[kTvT2], tz1[kTvT2], ty1[kTvT2];   // the same of the second, plane b
+  const int me = threadIdx.x, tx = me % g.tx, ty = me / g.tx;
+  const unsigned pos = xcd_position(blockIdx.x, gridDim.x), bx = pos % g.gx, byz = pos / g.gx;
+  const int x = (int)bx * (g.tx - 4) + tx - 2, y = (int)(byz % g.gy) * (g.ty - 4) + ty - 2;
+  const int z0 = (int)(byz / g.gy) * g.zc, z1 = min(z0 + g.zc, a.nz);
+  const bool mine = tx >= 2 && tx < g.tx - 2 && ty >= 2 && ty < g.ty - 2 && x < a.nx && y < a.ny;
+  auto wrap = [](int i, int n) {
+    i %= n;
+    return i < 0 ? i + n : i;
+  };
+  const int xw = wrap(x, a.nx), yw = wrap(y, a.ny);
+  const Off col = ((Off)yw * (Off)a.nx + (Off)xw) * (Off)sizeof(T);
+  const long long nxy = (long long)a.nx * a.ny, n = nxy * a.nz;
+  const int lx = me - (tx > 0), ly = ty > 0 ? me - g.tx : me;                          // lower neighbours
+  const int ux = me + (tx < g.tx - 1), uy = ty < g.ty - 1 ? me + g.tx : me;            // upper neighbours
+  const float c = 1.0f / (12.0f * a.lam);
+  const bool edge = a.dirichlet && (xw == 0 || yw == 0 || xw == a.nx - 1 || yw == a.ny - 1);
+  auto ld = [&](const T* plane) { return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(plane) + col); };
+  auto st = [&](T* plane, T v) { *reinterpret_cast<T*>(reinterpret_cast<char*>(plane) + col) = v; };
+  auto on_face = [&](int zw) { return edge || (a.dirichlet && (zw == 0 || zw == a.nz - 1)); };
+
+  int za = wrap(z0 - 2, a.nz), za1 = 0, zb = 0;    // planes a, a - 1 and b, wrapped
+  T p[3], o[3], vi;                                // P_k, P_{k-1} and in of plane a
+  T pn[3]{}, on[3]{}, vn{};                        // and of plane a + 1
+  constexpr int D = sizeof(T) == 4 ? 2 : 1;
+  int zn = za + 1 < a.nz ? za + 1 : 0;
+  auto request = [&](int z, T (&pz)[3], T (&oz)[3], T& vz) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      pz[k] = ld(Pc + k * n + z * nxy);
+      oz[k] = ld(Pp + k * n + z * nxy);
+    }
+    vz = ld(in + z * nxy);
+  };
+  request(za, p, o, vi);
+  if constexpr (D == 2) request(zn, pn, on, vn);
+  T pk[3]{}, vi_a1{}, vi_b{};                      // P_k and in of plane a - 1, in of plane b
+  T q0{}, q1{}, rz{}, y_a1{};                      // plane a - 1: R_x + c grad_x, R_y + c grad_y, R_z and y
+  T t[3]{}, u0{}, u1{}, tz{}, y_b1{};              // R of the second iteration, plane b; as above, plane b - 1
+  const int last = z1 - z0 + 4;
+  for (int s = 0; s <= last; ++s) {
+    // the first iteration is through a step before the last, the second one starts at s = 3
+    const bool one = s < last, two = s >= 3;
+    const int zm = zn + 1 < a.nz ? zn + 1 : 0;     // plane a + 2
+    T pm[3]{}, om[3]{}, vm{}, r[3]{}, v{}, w{};
+    if constexpr (D == 2) {
+      if (s + 2 < last) request(zm, pm, om, vm);
+    } else {
+      if (s + 1 < last) request(zn, pn, on, vn);
+    }
+    if (one) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) r[k] = p[k] + theta * (p[k] - o[k]);
+      sx[me] = r[0];
+      sz[me] = r[1];
+    }
+    if (two) {
+      tx1[me] = t[0];
+      tz1[me] = t[1];
+    }
+    lds_barrier();
+    if (one) {
+      v = tv_bounds(vi - a.lam * (((r[0] + r[1]) + r[2]) - sx[lx] - sz[ly] - rz), a);
+      if (on_face(za)) tv_zero_val(v);
+      sy[me] = v;
+    }
+    if (two) {
+      w = tv_bounds(vi_b - a.lam * (((t[0] + t[1]) + t[2]) - tx1[lx] - tz1[ly] - tz), a);
+      if (on_face(zb)) tv_zero_val(w);
+      ty1[me] = w;
+    }
+    lds_barrier();
+    const int a1 = z0 - 3 + s, b1 = z0 - 5 + s;    // planes a - 1 and b - 1
+    if (two) {
+      if (mine && b1 >= z0) {
+        const T m2 = tz + c * (y_b1 - w);
+        const float inv1 = tv_rsqrt(fmaxf(tv_abs2(u0) + tv_abs2(u1) + tv_abs2(m2), 1.0f));
+        st(P2 + b1 * nxy, inv1 * u0);
+        st(P2 + n + b1 * nxy, inv1 * u1);
+        st(P2 + 2 * n + b1 * nxy, inv1 * m2);
+      }
+      u0 = t[0] + c * (w - ty1[ux]);
+      u1 = t[1] + c * (w - ty1[uy]);
+      tz = t[2];
+      y_b1 = w;
+    }
+    if (one) {
+      if (s >= 2) {
+        const T p2 = rz + c * (y_a1 - v);
+        const float inv = tv_rsqrt(fmaxf(tv_abs2(q0) + tv_abs2(q1) + tv_abs2(p2), 1.0f));
+        const T n0 = inv * q0, n1 = inv * q1, n2 = inv * p2;
+        if (mine && a1 >= z0 && a1 < z1) {
+          st(P1 + a1 * nxy, n0);
+          st(P1 + n + a1 * nxy, n1);
+          st(P1 + 2 * n + a1 * nxy, n2);
+        }
+        t[0] = n0 + theta1 * (n0 - pk[0]);
+        t[1] = n1 + theta1 * (n1 - pk[1]);
+        t[2] = n2 + theta1 * (n2 - pk[2]);
+      }
+      q0 = r[0] + c * (v - sy[ux]);
+      q1 = r[1] + c * (v - sy[uy]);
+      rz = r[2];
+      y_a1 = v;
+    }
+    vi_b = vi_a1;
+    vi_a1 = vi;
+    vi = vn;
+    if constexpr (D == 2) vn = vm;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      pk[k] = p[k];
+      p[k] = pn[k];
+      o[k] = on[k];
+      if constexpr (D == 2) {
+        pn[k] = pm[k];
+        on[k] = om[k];
+      }
+    }
+    zb = za1;
+    za1 = za;
+    za = zn;
+    zn = zm;
+  }
+}
+
 __global__ void tv_div_project(const float* __restrict__ in, const float* __restrict__ Q, float* __restrict__ y,
                                TvArgs a) {
   tv_div_project_body(in, Q, y, a);
@@ -211,6 +358,52 @@ void tv_inner_real(hipStream_t st, const float* in, const float* Pc, const float
 void tv_inner_complex(hipStream_t st, const float2* in, const float2* Pc, const float2* Pp, float2* Pn,
                       const TvArgs& a, float theta, bool first) {
   launch_inner<float2>(st, in, Pc, Pp, Pn, a, theta, first);
+}
+
+// Tiles of tv_inner2 and whether it pays (gz > 0): columns of up to 60 in x and what the threads of a block
+// hold in y, shared out evenly, and the planes a block that take the least time.  Times in us, fitted to the
+// sizes above and to small ones: a launch of tv_inner2 3 and 1.2 a step (real, one block a CU), 1.75 (two
+// blocks) or 1.8 (complex); two launches of tv_inner 3.3 each and their bytes at 5.2 TB/s, 5.4 at least.
+// 60 x 70 x 40 complex keeps tv_inner (6.8 us an iteration; 7.4), real takes tv_inner2 (5.5; 5.4).
+TvTiles tv_tiles(const TvArgs& a, bool cplx) {
+  TvTiles g;
+  g.gx = (a.nx + 59) / 60;
+  g.tx = (a.nx + g.gx - 1) / g.gx + 4;
+  const int uy = kTvT2 / g.tx - 4;
+  g.gy = (a.ny + uy - 1) / uy;
+  g.ty = (a.ny + g.gy - 1) / g.gy + 4;
+  const long long cols = (long long)g.gx * g.gy, cus = 256;
+  double best = 0.0;
+  for (int zc = 1; zc <= a.nz; ++zc) {
+    const long long nb = cols * ((a.nz + zc - 1) / zc);
+    const bool two = !cplx && nb > cus;            // two blocks a CU
+    const long long rounds = two ? (nb + 2 * cus - 1) / (2 * cus) : (nb + cus - 1) / cus;
+    const double t = 3.0 + (double)rounds * (zc + 4) * (cplx ? 1.8 : two ? 1.75 : 1.2);
+    if (best > 0.0 && t >= best) continue;
+    best = t;
+    g.zc = zc;
+  }
+  g.gz = (a.nz + g.zc - 1) / g.zc;
+  const double bytes = 10.0 * (cplx ? 8.0 : 4.0) * a.nx * a.ny * a.nz;
+  if (best >= 2.0 * std::max(5.4, 3.3 + bytes / 5.2e6) || cols * g.gz >= (1ll << 31)) g.gz = 0;
+  return g;
+}
+template <class T>
+static void launch_inner2(hipStream_t st, const T* in, const T* Pc, const T* Pp, T* P1, T* P2, const TvArgs& a,
+                          const TvTiles& g, float theta, float theta1) {
+  const dim3 grid((unsigned)((long long)g.gx * g.gy * g.gz)), block((unsigned)(g.tx * g.ty));
+  if ((unsigned long long)a.nx * a.ny * sizeof(T) < (1ull << 32))
+    hipLaunchKernelGGL((tv_inner2<T, unsigned>), grid, block, 0, st, in, Pc, Pp, P1, P2, a, g, theta, theta1);
+  else
+    hipLaunchKernelGGL((tv_inner2<T, unsigned long long>), grid, block, 0, st, in, Pc, Pp, P1, P2, a, g, theta, theta1);
+}
+void tv_inner2_real(hipStream_t st, const float* in, const float* Pc, const float* Pp, float* P1, float* P2,
+                    const TvArgs& a, const TvTiles& g, float theta, float theta1) {
+  launch_inner2<float>(st, in, Pc, Pp, P1, P2, a, g, theta, theta1);
+}
+void tv_inner2_complex(hipStream_t st, const float2* in, const float2* Pc, const float2* Pp, float2* P1, float2* P2,
+                       const TvArgs& a, const TvTiles& g, float theta, float theta1) {
+  launch_inner2<float2>(st, in, Pc, Pp, P1, P2, a, g, theta, theta1);
 }
 
 __global__ void tv_zero(float* __restrict__ buf, long long n) {

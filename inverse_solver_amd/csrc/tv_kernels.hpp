@@ -9,6 +9,11 @@ struct TvArgs {
   int non_neg, dirichlet;
 };
 
+// Blocks of tv_inner2: gx x gy x gz of them, each of tx x ty threads and zc planes; gz = 0: tv_inner is faster.
+struct TvTiles {
+  int gx, gy, gz, tx, ty, zc;
+};
+
 // y = project(in - lam div(Q)) of a real potential (one float per voxel, the dual Q three) or a
 // complex one (complex64 per voxel).
 __global__ void tv_div_project(const float* __restrict__ in, const float* __restrict__ Q, float* __restrict__ y,
@@ -21,6 +26,13 @@ void tv_inner_real(hipStream_t st, const float* in, const float* Pc, const float
                    float theta, bool first);
 void tv_inner_complex(hipStream_t st, const float2* in, const float2* Pc, const float2* Pp, float2* Pn,
                       const TvArgs& a, float theta, bool first);
+// Two of them: P1 = P_{k+1} and P2 = P_{k+2} (apart from Pc, Pp and each other), with the momentum theta
+// between P_k and P_{k-1} and theta1 between P_{k+1} and P_k.
+void tv_inner2_real(hipStream_t st, const float* in, const float* Pc, const float* Pp, float* P1, float* P2,
+                    const TvArgs& a, const TvTiles& g, float theta, float theta1);
+void tv_inner2_complex(hipStream_t st, const float2* in, const float2* Pc, const float2* Pp, float2* P1, float2* P2,
+                       const TvArgs& a, const TvTiles& g, float theta, float theta1);
+TvTiles tv_tiles(const TvArgs& a, bool cplx);
 __global__ void tv_zero(float* __restrict__ buf, long long n);
 
 // Misfit gradient from the forward and adjoint 3D fields (n_rhs blocks of nx*ny*nz complex64).
