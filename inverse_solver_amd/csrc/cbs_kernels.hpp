@@ -181,6 +181,19 @@ __device__ __forceinline__ float2 born_step(int upd, int fwd, float2 q, float2 r
   return cmul(p, make_float2(r.x, sg_fwd * r.y));
 }
 
+// The dyadic Green's multiply G (I - c r r^T) of one frequency on its three components
+// (Codes/FORWARD_SOLVER_CONVERGENT_BORN.m:607-615): d = 4 pi^2 |k_s|^2 - k_m^2, r its direction over k0.
+__device__ __forceinline__ void dyadic_mul(const Consts& c, float d, float r0, float r1, float r2, float2& v0, float2& v1,
+                                           float2& v2) {
+  const float s = c.inv_n * __builtin_amdgcn_rcpf(fmaf(d, d, c.eps * c.eps));   // hardware reciprocal (1 ulp)
+  const float2 g = make_float2(d * s, c.eps * s);
+  const float2 dot = make_float2(r0 * v0.x + r1 * v1.x + r2 * v2.x, r0 * v0.y + r1 * v1.y + r2 * v2.y);
+  const float2 cd = cmul(make_float2(c.c_re, c.c_im), dot);
+  v0 = cmul(g, make_float2(v0.x - r0 * cd.x, v0.y - r0 * cd.y));
+  v1 = cmul(g, make_float2(v1.x - r1 * cd.x, v1.y - r1 * cd.y));
+  v2 = cmul(g, make_float2(v2.x - r2 * cd.x, v2.y - r2 * cd.y));
+}
+
 // Ramp orientation signs for born_step from the flip states (1 = Greenp flipped).
 __device__ __forceinline__ float sign_inv(int flip_inv) { return flip_inv ? 1.f : -1.f; }
 __device__ __forceinline__ float sign_fwd(int flip_fwd) { return flip_fwd ? -1.f : 1.f; }

@@ -816,6 +816,69 @@ __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb
   }
 }
 
+// The same for vector runs: a block holds the three components of its lines (component q's line l at index
+// q T + l of a row of the tile) and applies the dyadic factor of green_plain_vec between the transforms, where
+// the transforms and the factor on their own moved each component three times.  With the x passes fused as well,
+// 100 x 120 x 75 x 4 rhs of three components went from 375 to 200 us an iteration.
+template <int N, int T, int NT>
+__global__ __launch_bounds__(NT) void line_strided_green3(float2* data, Tables tb, Consts c, const float2* tw,
+                                                          const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+  constexpr int K = (N * T + NT - 1) / NT;
+  __shared__ float2 lds[3 * N * T];
+  __shared__ float2 s_tw[N];
+  const int ntile = (c.nx + T - 1) / T;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
+  const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / T) ny rhs blocks
+  if (cv.norms && conv_stopped(cv, jj - 1, r)) return;
+  const int flip = flip_of(jj, parity, 3 * r);
+  const int x0 = xt * T;
+  const int tv = c.nx - x0 < T ? c.nx - x0 : T;
+  const long long es = (long long)c.nx * c.ny;
+  float2* base = data + (long long)(3 * r) * c.nvox + (long long)y * c.nx + x0;
+  auto ad = [](int l, int e) { return e * 3 * T + l; };
+  float2 xv[3][K];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = threadIdx.x + k * NT;
+      const int e = i / T, t = i - e * T;
+      xv[q][k] = make_float2(0.f, 0.f);
+      if (i < N * T && t < tv) xv[q][k] = base[q * c.nvox + e * es + t];
+    }
+  for (int i = threadIdx.x; i < N; i += NT) s_tw[i] = tw[i];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = threadIdx.x + k * NT;
+      const int e = i / T, t = i - e * T;
+      if (i < N * T) lds[ad(q * T + t, e)] = xv[q][k];
+    }
+  __syncthreads();
+  const float* gx = tb.green_x + flip * c.nx + x0;
+  const float* gz = tb.green_z + flip * c.nz;
+  const float gy = tb.green_y[flip * c.ny + y];
+  const float* rx = tb.rad_x + flip * c.nx + x0;
+  const float* rz = tb.rad_z + flip * c.nz;
+  const float ry = tb.rad_y[flip * c.ny + y];
+  auto dyadic = [&](int l, int pz, float2& v0, float2& v1, float2& v2) {
+    const int t = l < tv ? l : 0;
+    dyadic_mul(c, gx[t] + gy + gz[pz] - c.km2, rx[t], ry, rz[pz], v0, v1, v2);
+  };
+  line_fft_mul3_ifft<N, T, NT>(lds, ad, s_tw, threadIdx.x, dyadic);
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = threadIdx.x + k * NT;
+      const int e = i / T, t = i - e * T;
+      if (i < N * T && t < tv) base[q * c.nvox + e * es + t] = lds[ad(q * T + t, e)];
+    }
+}
+
 // FFT along x for R rows per block (rows are contiguous nx-vectors).
 template <int NX, int ROWS, int NT>
 __global__ __launch_bounds__(NT) void fft_rows(float2* data, long long nrows, const float2* tw, int inverse) {

@@ -455,6 +455,54 @@ __global__ __launch_bounds__(NT) void dense_strided_green(float2* data, Tables t
   store_strided<KC, NT>(base, es, n, tv, tid, lds);
 }
 
+// The same for vector runs: the three components' tiles in LDS, the dyadic factor of green_plain_vec between
+// the transforms.  68 x 98 x 58 x 4 rhs of three components, with the x passes fused as well: 263 -> 145 us an
+// iteration (Bluestein's transforms and separate passes before).
+template <int KC, int NT, int TPW>
+__global__ __launch_bounds__(NT) void dense_strided_green3(float2* data, Tables tb, Consts c, DenseArgs p,
+                                                            const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+  extern __shared__ float2 s_tw[];
+  float2* lds = s_tw + dense_tables(p);
+  const int n = p.n, tid = threadIdx.x, tile = n * kL;
+  const int ntile = (c.nx + kL - 1) / kL;
+  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const int xt = bid % ntile;
+  const int o = bid / ntile;
+  const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / 16) ny rhs blocks
+  if (cv.norms && conv_stopped(cv, jj - 1, r)) return;
+  const int flip = flip_of(jj, parity, 3 * r);
+  const int x0 = xt * kL;
+  const int tv = c.nx - x0 < kL ? c.nx - x0 : kL;
+  const long long es = (long long)c.nx * c.ny;
+  float2* __restrict__ base = data + (long long)(3 * r) * c.nvox + (long long)y * c.nx + x0;
+  DenseTables<NT, tables_k(KC * NT / kL, NT)> tabs;
+  tabs.load(p, tid);
+  float2 va[KC], vb[KC];                         // two components are in flight
+  load_strided<KC, NT>(base, es, n, tv, tid, va);
+  load_strided<KC, NT>(base + c.nvox, es, n, tv, tid, vb);
+  tabs.store(s_tw, tid);
+  each_strided<KC, NT>(n, tid, [&](int k, int i) { lds[i] = va[k]; });
+  load_strided<KC, NT>(base + 2 * c.nvox, es, n, tv, tid, va);
+  each_strided<KC, NT>(n, tid, [&](int k, int i) { lds[tile + i] = vb[k]; });
+  each_strided<KC, NT>(n, tid, [&](int k, int i) { lds[2 * tile + i] = va[k]; });
+  lds_barrier();
+#pragma unroll 1
+  for (int q = 0; q < 3; ++q) dense_lines<kL, NT, TPW, false>(lds + q * tile, s_tw, p, tid);
+  const int tx = flip * c.nx + x0 + min(tid & 15, tv - 1);   // every element of a thread is in one column
+  const float gx = tb.green_x[tx], gy = tb.green_y[flip * c.ny + y], rx = tb.rad_x[tx], ry = tb.rad_y[flip * c.ny + y];
+  const float* __restrict__ gz = tb.green_z + flip * n;
+  const float* __restrict__ rz = tb.rad_z + flip * n;
+  each_strided<KC, NT>(n, tid, [&](int, int i) {
+    const int z = i >> 4;
+    dyadic_mul(c, gx + gy + gz[z] - c.km2, rx, ry, rz[z], lds[i], lds[tile + i], lds[2 * tile + i]);
+  });
+  lds_barrier();
+#pragma unroll 1
+  for (int q = 0; q < 3; ++q) dense_lines<kL, NT, TPW, true>(lds + q * tile, s_tw, p, tid);
+#pragma unroll 1
+  for (int q = 0; q < 3; ++q) store_strided<KC, NT>(base + q * c.nvox, es, n, tv, tid, lds + q * tile);
+}
+
 // (longest line, threads of the strided kernels, most tasks of a tile).  The strided kernels
 // take 256 threads where four waves hold the tasks: a CU then keeps twice the blocks, and with
 // them twice the waves that have work in the products.
@@ -466,7 +514,8 @@ constexpr int tasks_a_wave(int tasks, int nt) { return (tasks + nt / 64 - 1) / (
    {&dense_rows_update<N / 64, tasks_a_wave(TASKS, kNT), UPD_NONE>,                                                \
     &dense_rows_update<N / 64, tasks_a_wave(TASKS, kNT), UPD_DEFER>,                                               \
     &dense_rows_update<N / 64, tasks_a_wave(TASKS, kNT), UPD_PAIR>},                                               \
-   &dense_strided_green<N * kL / NT, NT, tasks_a_wave(TASKS, NT)>, N, TASKS, kNT, NT, kL},
+   &dense_strided_green<N * kL / NT, NT, tasks_a_wave(TASKS, NT)>,                                                 \
+   &dense_strided_green3<N * kL / NT, NT, tasks_a_wave(TASKS, NT)>, N, TASKS, kNT, NT, kL},
 static const DenseInfo kDense[] = {DENSE_LIST(DENSE_ENTRY)};
 
 const DenseInfo* find_dense(int n, int ntask) {

@@ -75,13 +75,14 @@ struct DenseInfo {
   DenseRowsFn rows;
   DenseStridedFn strided;
   DenseRowsUpdateFn rows_update[3];   // any launch; steady UPD_DEFER; steady UPD_PAIR
-  DenseStridedGreenFn strided_green;
+  DenseStridedGreenFn strided_green, strided_green3;   // one component; the three of a vector run
   int nmax, tasks;          // longest line, most tasks of a tile
   int nt_rows, nt_strided;  // threads of a block
   int lines;                // lines of a tile
   // dynamic LDS: the tables and the tile (rows: one word of padding an element)
   size_t lds_rows(const DenseArgs& a) const { return (size_t)(a.n * (lines + 1) + dense_tables(a)) * sizeof(float2); }
   size_t lds_strided(const DenseArgs& a) const { return (size_t)(a.n * lines + dense_tables(a)) * sizeof(float2); }
+  size_t lds_green3(const DenseArgs& a) const { return lds_strided(a) + (size_t)(2 * a.n * lines) * sizeof(float2); }
 };
 // the kernels for lines of n elements and ntask tasks (null: too long)
 const DenseInfo* find_dense(int n, int ntask);

@@ -60,7 +60,8 @@ using StridedGreenFn = void (*)(float2*, Tables, Consts, const float2*, const ui
 struct RowsUpdateInfo { RowsUpdateFn fn, fn_vr; int n, rows, nt; };   // fn_vr: real potential (st.Vr)
 struct StridedGreenInfo { StridedGreenFn fn; int n, t, nt; };
 const RowsUpdateInfo* find_rows_update(int n);
-const StridedGreenInfo* find_strided_green(int n);
+// pole: field components (3: the dyadic Green's function; null above 400 points)
+const StridedGreenInfo* find_strided_green(int n, int pole);
 // enumerate for planning
 int list_pass_real(const PassRInfo** out);
 int list_pass_kspace(const PassKInfo** out);

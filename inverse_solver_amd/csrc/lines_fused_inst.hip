@@ -20,17 +20,27 @@ constexpr int fused_t(int n) { return n <= 576 ? 16 : 8; }
 #define RU_ENTRY(N) {&line_rows_update<N, fused_rows(N), 256, 0>, &line_rows_update<N, fused_rows(N), 256, 1>, N, fused_rows(N), 256},
 #define SG_ENTRY(N) {&line_strided_green<N, fused_t(N), 256>, N, fused_t(N), 256},
 
+// vector runs: three components of up to 400 points, 78 KB of LDS and less
+constexpr int vec_t(int n) { return n <= 200 ? 16 : 8; }
+template <int N>
+constexpr StridedGreenInfo vec_entry() {
+  if constexpr (N <= 400) return {&line_strided_green3<N, vec_t(N), 256>, N, vec_t(N), 256};
+  else return {nullptr, N, 0, 0};
+}
+#define SG3_ENTRY(N) vec_entry<N>(),
+
 static const RowsUpdateInfo kRU[] = {FUSED_LIST(RU_ENTRY)};
 static const StridedGreenInfo kSG[] = {FUSED_LIST(SG_ENTRY)};
+static const StridedGreenInfo kSG3[] = {FUSED_LIST(SG3_ENTRY)};
 
 const RowsUpdateInfo* find_rows_update(int n) {
   for (const auto& e : kRU)
     if (e.n == n) return &e;
   return nullptr;
 }
-const StridedGreenInfo* find_strided_green(int n) {
-  for (const auto& e : kSG)
-    if (e.n == n) return &e;
+const StridedGreenInfo* find_strided_green(int n, int pole) {
+  for (const auto& e : (pole == 3 ? kSG3 : kSG))
+    if (e.n == n && e.fn) return &e;
   return nullptr;
 }
 

@@ -1012,17 +1012,21 @@ struct Solver {
       else if (axis == 1) fy();
       else fz();
     };
-    // single-component runs: the x inverse, the update and the x forward (the z forward, the
-    // Green's multiply and the z inverse) run as one launch each, on compiled line lengths
-    // (lines_fused_inst.hip), matrix-core products (fft_dense.hip) or Bluestein's transform on a
-    // compiled length (fft_blue.hip)
-    const bool fuse = P == 1 && plan.form == CBS_FORM_PLAIN;   // CBS_FORM_AXES: every pass on its own
-    const BlueInfo* bx = (fuse && plan.rt[0]) ? rtp[0].bi : nullptr;
-    const BlueInfo* bz = (fuse && plan.rt[2]) ? rtp[2].bi : nullptr;
+    // the x inverse, the update and the x forward (the z forward, the Green's multiply and the z
+    // inverse) run as one launch each, on compiled line lengths (lines_fused_inst.hip), matrix-core
+    // products (fft_dense.hip) or, single-component runs, Bluestein's transform on a compiled length
+    // (fft_blue.hip).  Vector runs hold the three components of a z line in LDS.
+    const bool fuse = plan.form == CBS_FORM_PLAIN;   // CBS_FORM_AXES: every pass on its own
+    const BlueInfo* bx = (fuse && P == 1 && plan.rt[0]) ? rtp[0].bi : nullptr;
+    const BlueInfo* bz = (fuse && P == 1 && plan.rt[2]) ? rtp[2].bi : nullptr;
     const DenseInfo* dx = (fuse && plan.rt[0]) ? rtp[0].di : nullptr;
     const DenseInfo* dz = (fuse && plan.rt[2]) ? rtp[2].di : nullptr;
+    // three tiles of matrix-core transforms while two blocks share a CU's LDS, up to about 205 points: 194 points
+    // 198 us an iteration (separate passes 202), 249 points 297 (241).  Compiled lengths gain up to
+    // 400 points (300 points: 218; 251).
+    if (dz && P == 3 && dz->lds_green3(rtp[2].da) > 81920) dz = nullptr;
     const RowsUpdateInfo* cx = (fuse && !plan.rt[0]) ? find_rows_update(nx) : nullptr;
-    const StridedGreenInfo* cz = (fuse && !plan.rt[2]) ? find_strided_green(nz) : nullptr;
+    const StridedGreenInfo* cz = (fuse && !plan.rt[2]) ? find_strided_green(nz, P) : nullptr;
     const long long rows = (long long)ny * nz;
     require(rows < (1ll << 31), CBS_ERR_UNSUPPORTED, "grid too large for the per-axis passes");
     auto xpass = [&](int upd, int fwd, int jj_inv, int jj_fwd) {   // (x inverse,) update(, x forward)
@@ -1050,17 +1054,18 @@ struct Solver {
     };
     auto zpass = [&](int jj) {   // z forward, Green's multiply, z inverse
       if (cz) {
-        const long long nblk = (long long)((nx + cz->t - 1) / cz->t) * ny * nv;
+        const long long nblk = (long long)((nx + cz->t - 1) / cz->t) * ny * nb;
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
         timed(2, [&] { hipLaunchKernelGGL(cz->fn, dim3((unsigned)nblk), dim3(cz->nt), 0, stream, ws.spec, tb, c,
                                           tabs.tw_z.p, ws.parity, jj, cv); });
         return;
       }
       if (dz) {
-        const long long nblk = (long long)((nx + dz->lines - 1) / dz->lines) * ny * nv;
+        const long long nblk = (long long)((nx + dz->lines - 1) / dz->lines) * ny * nb;
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
-        timed(2, [&] { hipLaunchKernelGGL(dz->strided_green, dim3((unsigned)nblk), dim3(dz->nt_strided),
-                                          dz->lds_strided(rtp[2].da), stream, ws.spec, tb, c, rtp[2].da, ws.parity, jj,
+        const size_t lds = P == 3 ? dz->lds_green3(rtp[2].da) : dz->lds_strided(rtp[2].da);
+        timed(2, [&] { hipLaunchKernelGGL(P == 3 ? dz->strided_green3 : dz->strided_green, dim3((unsigned)nblk),
+                                          dim3(dz->nt_strided), lds, stream, ws.spec, tb, c, rtp[2].da, ws.parity, jj,
                                           cv); });
         return;
       }
@@ -2082,8 +2087,7 @@ struct Solver {
   // a real RI's potential is read as Vr by the real-space passes and the x transforms fused with the update:
   // 4 bytes a voxel less of 40 or 56 (576^2 x 320 x 4 rhs 527.8 -> 523.1 ms, 263 x 238 x 129 x 6 40.8 -> 40.0)
   bool has_vr() const {
-    return v_real && (plan.form == CBS_FORM_FUSED || plan.form == CBS_FORM_ROWS ||
-                      (plan.form == CBS_FORM_PLAIN && P == 1));
+    return v_real && plan.form != CBS_FORM_AXES;
   }
   // Vt (the fused plan's a and b) or Vr from the current V
   void sync_vtile() {
