@@ -330,7 +330,7 @@ struct Solver {
   // the potential or the plan changes, never inside a solve: the fused form's Vt, or for a real RI (V's
   // imaginary part -eps everywhere, as potential_fill forms it) only its real part, Vr
   DevBuf<float2> Vt;
-  DevBuf<float> Vr;
+  float* vr() const { return reinterpret_cast<float*>(V.p + (nvox + 31) / 32 * 32); }   // behind V, one allocation
   bool v_real = false;
   long long v_version = 0;
   std::vector<long long> vt_key;
@@ -825,7 +825,7 @@ struct Solver {
     (void)nb;
     StateArgs s;
     s.V = plan.form == CBS_FORM_FUSED && !v_real ? Vt.p : V.p;
-    s.Vr = has_vr() ? Vr.p : nullptr;
+    s.Vr = has_vr() ? vr() : nullptr;
     s.field = ws.field; s.fstate = ws.fstate; s.spec = ws.spec; s.parity = ws.parity;
     s.rhs_stride = nvox;
     s.norms = nullptr;
@@ -2076,7 +2076,7 @@ struct Solver {
     prm = *p;
     drop_graph();
     v_real = cplx == 0;   // Im V = 0 - eps at every voxel, inside the RI grid and in the boundary
-    V.ensure((size_t)nvox);
+    V.ensure((size_t)((nvox + 31) / 32 * 32 + (v_real ? (nvox + 1) / 2 : 0)));   // Vr behind it
     const RoiGeom rg = roi();
     hipLaunchKernelGGL(potential_fill, dim3(grid_for(nvox)), dim3(256), 0, stream, g, flip_conj, rg, nx, ny,
                        (long long)nvox, p->eps_imag, V.p);
@@ -2096,8 +2096,7 @@ struct Solver {
                                         (long long)v_real};
     if (key == vt_key) return;
     if (v_real) {
-      Vr.ensure((size_t)nvox);
-      hipLaunchKernelGGL(tile_rows_real, dim3(grid_for(nvox)), dim3(256), 0, stream, V.p, Vr.p, consts(1));
+      hipLaunchKernelGGL(tile_rows_real, dim3(grid_for(nvox)), dim3(256), 0, stream, V.p, vr(), consts(1));
     } else {
       Vt.ensure((size_t)nvox);
       hipLaunchKernelGGL(tile_rows, dim3(grid_for(nvox)), dim3(256), 0, stream, V.p, Vt.p, consts(1));
