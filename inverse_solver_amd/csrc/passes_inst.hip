@@ -15,7 +15,7 @@ namespace cbs {
   X(96, 96, 256) X(96, 96, 512) X(96, 48, 256) X(96, 48, 512) X(96, 32, 256) X(96, 24, 256) X(96, 24, 576) \
   X(128, 64, 256) X(128, 64, 512) X(128, 32, 256) X(128, 32, 512) \
   X(160, 40, 256) X(160, 40, 512) X(160, 32, 256) X(160, 32, 512) X(160, 20, 256) X(160, 80, 512) \
-  X(192, 48, 256) X(192, 48, 512) X(192, 32, 256) \
+  X(192, 48, 256) X(192, 48, 512) X(192, 48, 768) X(192, 32, 256) \
   X(288, 32, 256) X(288, 32, 512)
 
 // four-pass form (contiguous row blocks, y and z transforms in their own passes): (NX, rows, NT)
@@ -27,7 +27,7 @@ namespace cbs {
   X(1, 32, 16, 256) X(2, 32, 16, 256) X(1, 40, 16, 256) X(2, 40, 16, 256) X(2, 40, 8, 192) X(1, 30, 8, 256) X(1, 36, 8, 256) \
   X(1, 96, 32, 256) X(1, 96, 32, 512) X(1, 96, 16, 256) X(2, 96, 16, 256) X(2, 96, 32, 512) X(3, 96, 16, 256) \
   X(2, 96, 8, 256) X(3, 96, 8, 256) X(4, 96, 8, 256) X(4, 96, 16, 256) X(4, 96, 16, 512) X(4, 96, 4, 256) \
-  X(2, 135, 32, 256) X(2, 135, 32, 512) X(2, 135, 16, 256) X(4, 135, 8, 256) X(4, 135, 16, 512) X(4, 135, 16, 768) \
+  X(2, 135, 32, 256) X(2, 135, 32, 512) X(2, 135, 32, 768) X(2, 135, 16, 256) X(4, 135, 8, 256) X(4, 135, 16, 512) X(4, 135, 16, 768) \
   X(2, 128, 32, 256) X(4, 128, 16, 256) X(4, 128, 16, 512) X(6, 128, 8, 256) X(4, 128, 8, 256) \
   X(4, 160, 16, 256) X(4, 160, 16, 512) X(4, 160, 16, 768) X(4, 160, 16, 1024) X(5, 160, 8, 256) X(8, 160, 8, 256) X(4, 160, 8, 256) \
   X(2, 160, 32, 512) X(2, 160, 32, 256) \

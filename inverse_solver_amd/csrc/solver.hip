@@ -525,7 +525,8 @@ struct Solver {
       // Vector runs, and runs whose transforms keep their rounding (cbs_set_transforms): the largest a
       // whose tile keeps two blocks per CU (<= 80 KiB); vector runs then the narrowest x tile of 16 and more.
       // Threads: real space 512 for tiles of 32 KiB and more (128 x 32, 24 rhs: 14.8 against
-      // 15.1 us on 256), else 256; k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 26.1 against 27.4
+      // 15.1 us on 256), else 256; 768 where listed, for tiles whose transforms' tasks it divides better (192 x 48:
+      // 768 to 1536 tasks a step; 12 rhs of 192^2 x 128 638 -> 620 us an iteration; 160 x 40 took 61 for 59); k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 26.1 against 27.4
       // on 512 and 32.3 on 1024), 512 from 40 KiB (96^3 x 24: 2.8; 768 threads 3.1, 256 3.1).
       const bool keep = P > 1 || !dense;
       auto score_r = [&](const PassRInfo& r) {
@@ -533,7 +534,7 @@ struct Solver {
         bool wide = false;   // a 16-wide x tile with this b
         for (int j = 0; j < npk; ++j) wide = wide || (fused_ok_k(pks[j], b) && pks[j].t >= 16);
         const int pref = keep ? r.a * 10 : wide && b <= 4 && r.a * r.nx >= 2048 ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
-        return (r.lds <= 81920 ? 1000000 : 0) + pref + (r.nt == (r.lds >= 32768 ? 512 : 256) ? 1 : 0);
+        return (r.lds <= 81920 ? 1000000 : 0) + pref + (r.nt == 768 ? 2 : r.nt == (r.lds >= 32768 ? 512 : 256) ? 1 : 0);
       };
       auto score_k = [&](const PassKInfo& q) {
         const int want = P > 1 ? 512 : q.lds >= 64000 ? 768 : 512;
