@@ -524,10 +524,11 @@ struct Solver {
       // CU) 741, 4-wide (32-byte rows) 808.  160^3 and 192^2 x 128 have b = 4 either way.
       // Vector runs, and runs whose transforms keep their rounding (cbs_set_transforms): the largest a
       // whose tile keeps two blocks per CU (<= 80 KiB); vector runs then the narrowest x tile of 16 and more.
-      // Threads: real space 512 for tiles of 32 KiB and more (128 x 32, 24 rhs: 14.8 against
-      // 15.1 us on 256), else 256; 768 where listed, for tiles whose transforms' tasks it divides better (192 x 48:
-      // 768 to 1536 tasks a step; 12 rhs of 192^2 x 128 638 -> 620 us an iteration; 160 x 40 took 61 for 59); k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 26.1 against 27.4
-      // on 512 and 32.3 on 1024), 512 from 40 KiB (96^3 x 24: 2.8; 768 threads 3.1, 256 3.1).
+      // Threads: real space 512 for tiles of 32 KiB and more (128 x 32, 24 rhs: 361 us a launch against
+      // 367 on 256), else 256; 768 where listed, for tiles whose transforms' tasks it divides better (192 x 48: 768
+      // to 1536 tasks a step, 12 rhs of 192^2 x 128 638 -> 620 us an iteration; 160 x 40, 49 rhs took 1.49 ms a launch
+      // for 1.44); k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 0.65 ms a launch against 0.68 on
+      // 512 and 0.80 on 1024), 512 from 40 KiB (96^3 x 24: 70 us; 77 on 768 and on 256).
       const bool keep = P > 1 || !dense;
       auto score_r = [&](const PassRInfo& r) {
         const int b = ny / r.a;
