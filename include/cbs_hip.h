@@ -310,7 +310,8 @@ int cbs_set_convergence(cbs_handle h, double tol);
 /* Transforms of line lengths without a compiled FFT (prime factors above 5), in the per-axis form and
  * the 2D grids.  CBS_TRANSFORMS_FASTEST (the default): the matrix-core products up to 448 points.
  * CBS_TRANSFORMS_FIXED: Bluestein's transform and the run-time stages, whose rounding does not
- * change with the library, and the fused form's planner and cbs_autotune keep to one split of y:
+ * change with the library, and the fused form's planner and cbs_autotune keep to one split of y, and
+ * vector runs of the per-axis form keep their passes apart:
  * for callers that compare results bit for bit with earlier ones, as BACKWARD_SOLVER_MULTI's FP64
  * gradient is.  No counterpart in the reference, which plans cuFFT. */
 enum { CBS_TRANSFORMS_FASTEST = 0, CBS_TRANSFORMS_FIXED = 1 };

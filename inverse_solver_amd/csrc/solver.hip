@@ -1018,7 +1018,8 @@ struct Solver {
     // inverse) run as one launch each, on compiled line lengths (lines_fused_inst.hip), matrix-core
     // products (fft_dense.hip) or, single-component runs, Bluestein's transform on a compiled length
     // (fft_blue.hip).  Vector runs hold the three components of a z line in LDS.
-    const bool fuse = plan.form == CBS_FORM_PLAIN;   // CBS_FORM_AXES: every pass on its own
+    // CBS_FORM_AXES: every pass on its own; so do vector runs whose transforms keep their rounding (cbs_set_transforms)
+    const bool fuse = plan.form == CBS_FORM_PLAIN && (P == 1 || dense);
     const BlueInfo* bx = (fuse && P == 1 && plan.rt[0]) ? rtp[0].bi : nullptr;
     const BlueInfo* bz = (fuse && P == 1 && plan.rt[2]) ? rtp[2].bi : nullptr;
     const DenseInfo* dx = (fuse && plan.rt[0]) ? rtp[0].di : nullptr;

@@ -36,3 +36,19 @@ def test_vector_axes(ri, tol):
         err = rel(out[0], ref)
         print(ri, 'rel err', err, flush=True)
         assert err <= 1e-5
+
+
+def test_fixed_transforms_keep_the_separate_passes():
+    """cbs_set_transforms(FIXED): a vector run's fields are those of the separate passes bit for bit."""
+    from inverse_solver_amd import FORWARD_SOLVER_CONVERGENT_BORN, _lib
+    ri = (17, 17, 19)
+    p = params(ri, bt_px_target=4, iterations=6, vector_simulation=True)
+    u = np.stack([np.stack([random_field(ri, j) for j in range(3)], axis=-1)], axis=-1)
+    out = []
+    for form in (1, 3):
+        s = FORWARD_SOLVER_CONVERGENT_BORN(p, options=dict(form=form))
+        _lib.check(_lib.lib.cbs_set_transforms(s._h, _lib.CBS_TRANSFORMS_FIXED))
+        s.set_RI(sphere_ri(ri, 0.5, n_s=1.42))
+        out.append(s.solve_incident(u))
+        s.close()
+    np.testing.assert_array_equal(out[0], out[1])
