@@ -679,6 +679,9 @@ struct Solver {
   void build_tables() {
     drop_graph();   // captured loops hold the table addresses, which may move here
     tab_key.clear();
+    // nothing to solve with if a table or the plan's copy of V cannot be allocated
+    const bool had_potential = have_potential;
+    have_potential = false;
     const int a = plan.a, b = plan.b;
     TableSet& T = tabs;
     T.a = a; T.b = b;
@@ -787,6 +790,7 @@ struct Solver {
     }
     tab_key = table_key();
     sync_vtile();
+    have_potential = had_potential;
   }
 
   // ---- kernel timing
@@ -1885,6 +1889,7 @@ struct Solver {
       opt = saved;
       (void)hipEventDestroy(e0);
       (void)hipEventDestroy(e1);
+      have_potential = true;   // V is whole; build_tables takes it back if the tables are not
       make_plan();
       build_tables();
       throw;
@@ -2024,6 +2029,7 @@ struct Solver {
     require(p != nullptr && v != nullptr, CBS_ERR_ARG, "null potential argument");
     require(mem == CBS_MEM_HOST || mem == CBS_MEM_DEVICE, CBS_ERR_ARG, "mem must be CBS_MEM_HOST or CBS_MEM_DEVICE");
     check_params(p);
+    have_potential = false;   // until V is whole again (an allocation can fail)
     prm = *p;
     drop_graph();
     v_real = false;   // a caller's V is taken as complex
@@ -2076,6 +2082,7 @@ struct Solver {
     require(flip_conj == 0 || flip_conj == 1, CBS_ERR_ARG, "flip_conj must be 0 or 1");
     check_params(p);
     const RiGrid g = ri_grid(ri, cplx, wavelength, n_m, mem);
+    have_potential = false;   // until V is whole again: a real RI after a complex one makes it grow, and that can fail
     prm = *p;
     drop_graph();
     v_real = cplx == 0;   // Im V = 0 - eps at every voxel, inside the RI grid and in the boundary

@@ -1,0 +1,56 @@
+"""GPU: a set_RI that runs out of device memory.  A real RI after a complex one makes the potential's buffer grow; if
+that fails, the handle has no potential: solves are refused until the next set_RI that succeeds."""
+import numpy as np
+import pytest
+
+from helpers import params
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def _take_memory(leave):
+    """Device memory held but for about ``leave`` bytes."""
+    import torch
+    hold, size = [], torch.cuda.mem_get_info()[0] - leave
+    while size >= 8 * MB:
+        try:
+            hold.append(torch.empty(size, dtype=torch.uint8, device='cuda'))
+            size = torch.cuda.mem_get_info()[0] - leave
+        except torch.cuda.OutOfMemoryError:
+            size //= 2
+    return hold
+
+
+def test_failed_growth_leaves_no_potential():
+    import torch
+    from inverse_solver_amd import FORWARD_SOLVER_CONVERGENT_BORN, _lib
+    ri = (312, 312, 312)                    # 320^3: V is 262 MB of complex64, 393 MB with the real part behind it
+    p = params(ri, iterations=2)
+    RI = np.full(ri, 1.336)
+    RI[100:200, 100:200, 100:200] = 1.38
+    u = np.ones(ri, np.complex64)
+    s = FORWARD_SOLVER_CONVERGENT_BORN(p)
+    s.set_RI(RI + 1j * 1e-3 * (RI > 1.35))
+    s.solve_incident(u)                     # the state buffers are there before memory is taken
+    hold = _take_memory(64 * MB)
+    try:
+        if torch.cuda.mem_get_info()[0] > 100 * MB:       # V (262 MB) is given back before the new one is asked for
+            pytest.skip('device memory could not be taken')
+        with pytest.raises(_lib.CbsError) as e:
+            s.set_RI(RI)
+        assert e.value.code == _lib.CBS_ERR_MEMORY
+        with pytest.raises(_lib.CbsError) as e:
+            s.solve_incident(u)
+        assert e.value.code == _lib.CBS_ERR_STATE
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+    s.set_RI(RI)
+    got = s.solve_incident(u)
+    t = FORWARD_SOLVER_CONVERGENT_BORN(p)
+    t.set_RI(RI)
+    np.testing.assert_array_equal(got, t.solve_incident(u))
+    s.close()
+    t.close()
