@@ -310,8 +310,9 @@ int cbs_set_convergence(cbs_handle h, double tol);
 /* Transforms of line lengths without a compiled FFT (prime factors above 5), in the per-axis form and
  * the 2D grids.  CBS_TRANSFORMS_FASTEST (the default): the matrix-core products up to 448 points.
  * CBS_TRANSFORMS_FIXED: Bluestein's transform and the run-time stages, whose rounding does not
- * change with the library, and the fused form's planner and cbs_autotune keep to one split of y, and
- * vector runs of the per-axis form keep their passes apart:
+ * change with the library; the fused form's planner and cbs_autotune keep to one split of y (a split that
+ * cbs_autotune measured before, and the options that came with it, are dropped; one that the caller sets
+ * stays); and vector runs of the per-axis form keep their passes apart:
  * for callers that compare results bit for bit with earlier ones, as BACKWARD_SOLVER_MULTI's FP64
  * gradient is.  No counterpart in the reference, which plans cuFFT. */
 enum { CBS_TRANSFORMS_FASTEST = 0, CBS_TRANSFORMS_FIXED = 1 };

@@ -386,6 +386,9 @@ struct Solver {
   RtPlan rtp[3], io_rtx, io_rty;
 
   bool dense = true;              // lengths without a compiled FFT: matrix-core products (cbs_set_transforms)
+  // the options that cbs_autotune chose among every split of y, and those it found (cbs_set_transforms puts them back)
+  bool tuned = false;
+  cbs_options tuned_opt{}, untuned_opt{};
 
   void build_io_rt() {            // convolution-grid lengths without a compiled kernel: run-time plans
     if (!io_rows) build_rt(io_rtx, cx, dense);
@@ -396,6 +399,19 @@ struct Solver {
     HIP_CHECK(hipStreamSynchronize(stream));
     dense = kind == CBS_TRANSFORMS_FASTEST;
     drop_graph();
+    // a measured split is not the one that FIXED keeps to; one that the caller has set since stays
+    if (!dense && tuned && opt.form == tuned_opt.form && opt.split_a == tuned_opt.split_a &&
+        opt.tile_t == tuned_opt.tile_t && opt.threads_real == tuned_opt.threads_real &&
+        opt.threads_kspace == tuned_opt.threads_kspace) {
+      opt.form = untuned_opt.form;
+      opt.split_a = untuned_opt.split_a;
+      opt.tile_t = untuned_opt.tile_t;
+      opt.threads_real = untuned_opt.threads_real;
+      opt.threads_kspace = untuned_opt.threads_kspace;
+      if (opt.block_order == tuned_opt.block_order) opt.block_order = untuned_opt.block_order;
+      if (opt.max_batch == tuned_opt.max_batch) opt.max_batch = untuned_opt.max_batch;
+    }
+    tuned = false;
     ffp.nx = ffp.ny = 0;
     if (io.ready) build_io_rt();
     if (have_potential) {
@@ -1909,6 +1925,9 @@ struct Solver {
     opt.time_kernels = saved_time;
     opt.track_norms = saved_norm;
     conv_tol = saved_tol;
+    tuned = dense;
+    tuned_opt = opt;
+    untuned_opt = saved;
     plan = best_plan;
     build_tables();
     HIP_CHECK(hipStreamSynchronize(stream));
