@@ -124,8 +124,8 @@ struct Plan {
   int a = 0, b = 0, t = 0;
   const PassRInfo* pr = nullptr;
   const PassKInfo* pk = nullptr;
-  const PassRInfo* pr_few = nullptr;   // fused form: the passes of launches with few blocks (run_fused)
-  const PassKInfo* pk_few = nullptr;
+  const PassRInfo* pr_few = nullptr;   // fused form: the real-space pass of launches with few blocks (run_fused)
+  bool few_k = false;                  // and whether such a launch may take another k-space pass (few_kspace)
   const RowsInfo* rw = nullptr;
   const StridedInfo* sy = nullptr;
   const StridedInfo* sz = nullptr;
@@ -531,13 +531,21 @@ struct Solver {
       const PassKInfo* pks = nullptr;
       const int npk = list_pass_kspace(&pks);
       // default preference; cbs_autotune replaces it by measurement.
-      // Scalar runs: the largest b <= 4 whose real-space tile still holds 2048 points and whose
-      // k-space tile can be 16 wide, else b = 2; then an x tile of 8 and more that divides nx, 32 wide
-      // for b <= 2 and 16 wide above.  Iterations, us, of 1, 4 and 24 rhs at 96^3: b = 1 (largest
+      // Scalar runs: b = 4, else 2, else 1 where the real-space tile still holds 2048 points and the k-space
+      // tile can be 16 wide, else b = 2.  Iterations, us, of 1, 4 and 24 rhs at 96^3: b = 1 (largest
       // a) 32, 50, 245; b = 2 24.2, 44.3, 229; b = 4 23.9, 44.7, 227; at 128^2 x 135: b = 2 42.6, 119, 590;
-      // b = 4 36.4, 106, 555; of 1 and 16 rhs at 40^3 (8-wide tiles, 16-wide ones run past the row):
-      // b = 1 13.1, 27.4; b = 2 10.3, 23.1; of 4 rhs at 288^2 x 160, b = 9: 8-wide (92 KB, one block a
-      // CU) 741, 4-wide (32-byte rows) 808.  160^3 and 192^2 x 128 have b = 4 either way.
+      // b = 4 36.4, 106, 555; of 1 and 16 rhs at 40^3: b = 1 13.1, 27.4; b = 2 10.3, 23.1.  160^3 and
+      // 192^2 x 128 have b = 4 either way.  Two exceptions:
+      //  - z planes of up to 1024 points keep b = 1 from 64 planes on and where b = 2 has no 8-wide x tile (16 rhs
+      //    of 32^2 x 96 26.1 us, b = 2 30.8; one of 32^3 9.2, 9.8; but one of 32^2 x 40 10.0, b = 2 9.4);
+      //  - b = 4 with a not a multiple of 8 gives way to b = 2 where that has an 8-wide tile: neighbouring x tiles
+      //    are a blocks apart, and only whole multiples of the 8 XCDs put them on one, which then holds
+      //    their common lines (160 x 80 x 96, a = 20 and 40: one rhs 37.5, 30.1, four 64.2, 58.1).
+      // The x tile: 8 and more, 32 wide for b = 2 (16 rhs of 128 x 64 x 96 136 us, 16 wide 138), else 16
+      // (16 rhs of 40 x 20 x 320, b = 1: 54.5 us; 63.3 with 32), and one that divides nx, but not 8 for b = 1 or from
+      // 40 KiB on, where threads gain more than padding costs (16 rhs of 40 x 20 x 24 12.7 us, 8-wide 13.9; one
+      // of 24 x 96 x 160 18.1 us, 8-wide 21.0); of 4 rhs at 288^2 x 160, b = 9: 8-wide (92 KB, one block a
+      // CU) 741, 4-wide (32-byte rows) 808.
       // Vector runs, and runs whose transforms keep their rounding (cbs_set_transforms): the largest a
       // whose tile keeps two blocks per CU (<= 80 KiB); vector runs then the narrowest x tile of 16 and more.
       // Threads: real space 512 for tiles of 32 KiB and more (128 x 32, 24 rhs: 361 us a launch against
@@ -546,18 +554,25 @@ struct Solver {
       // for 1.44); k-space 768 for tiles of 64 KB and more (160^3 x 49 rhs: 0.65 ms a launch against 0.68 on
       // 512 and 0.80 on 1024), 512 from 40 KiB (96^3 x 24: 70 us; 77 on 768 and on 256).
       const bool keep = P > 1 || !dense;
+      bool eight = false;   // an 8-wide x tile with b = 2
+      for (int i = 0; i < npr; ++i)
+        for (int j = 0; j < npk; ++j)
+          eight = eight || (fused_ok_r(prs[i]) && 2 * prs[i].a == ny && fused_ok_k(pks[j], 2) && pks[j].t == 8);
       auto score_r = [&](const PassRInfo& r) {
         const int b = ny / r.a;
         bool wide = false;   // a 16-wide x tile with this b
         for (int j = 0; j < npk; ++j) wide = wide || (fused_ok_k(pks[j], b) && pks[j].t >= 16);
-        const int pref = keep ? r.a * 10 : wide && b <= 4 && r.a * r.nx >= 2048 ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
+        const bool whole = b == 1 && nx * ny <= 1024 && (nz >= 64 || !eight);
+        const bool held = wide && (b <= 2 || b == 4) && r.a * r.nx >= 2048 && !(b == 4 && r.a % 8 != 0 && eight);
+        const int pref = keep ? r.a * 10 : whole ? 6000 : held ? 5000 + 10 * b : b == 2 ? 4000 : r.a * 10;
         return (r.lds <= 81920 ? 1000000 : 0) + pref + (r.nt == 768 ? 2 : r.nt == (r.lds >= 32768 ? 512 : 256) ? 1 : 0);
       };
       auto score_k = [&](const PassKInfo& q) {
         const int want = P > 1 ? 512 : q.lds >= 64000 ? 768 : 512;
         const int nt = q.lds < 40960 ? (q.nt < 512 ? 1 : 0) : q.nt == want ? 2 : q.nt == 512 ? 1 : 0;
-        return 4 * ((P == 1 && q.t >= 8 ? 2000 : 0) + (q.lds <= 81920 ? 1000 : 0) +
-                    (P == 1 && nx % q.t == 0 ? 200 : 0) + (q.t >= 16 ? 100 : 0) + (P == 1 && q.b <= 2 ? q.t : -q.t)) + nt;
+        const bool divides = P == 1 && nx % q.t == 0 && (q.t >= 16 || (q.b > 1 && q.lds < 40960));
+        return 4 * ((P == 1 && q.t >= 8 ? 2000 : 0) + (q.lds <= 81920 ? 1000 : 0) + (divides ? 200 : 0) +
+                    (q.t >= 16 ? 100 : 0) + (P == 1 && q.b == 2 ? q.t : -q.t)) + nt;
       };
       long best = -1;
       for (int i = 0; i < npr; ++i) {
@@ -582,17 +597,14 @@ struct Solver {
         p.a = p.pr->a;
         p.b = ny / p.a;
         p.t = p.pk->t;
-        // Launches of few blocks (run_fused): the real-space variant with the most threads, the narrowest
-        // k-space tile of 4 and more.  One rhs of 96^3: 27.5 -> 23.9 us an iteration (576 threads 2.4 us
-        // of it), of 40^3 10.7 -> 10.3; at 4 rhs the wide forms are as fast or faster.
+        // Launches of few blocks (run_fused): the real-space variant with the most threads; k-space: few_kspace.
+        // One rhs of 96^3: 27.5 -> 23.9 us an iteration (576 threads 2.4 us of it), of 40^3 10.7 -> 10.3; at
+        // 4 rhs the wide forms are as fast or faster.
         p.pr_few = p.pr;
-        p.pk_few = p.pk;
+        p.few_k = P == 1 && opt.threads_kspace == 0 && opt.tile_t == 0;
         if (opt.threads_real == 0)
           for (int i = 0; i < npr; ++i)
             if (fused_ok_r(prs[i]) && prs[i].a == p.a && prs[i].nt > p.pr_few->nt) p.pr_few = &prs[i];
-        if (P == 1 && opt.threads_kspace == 0 && opt.tile_t == 0)
-          for (int j = 0; j < npk; ++j)
-            if (fused_ok_k(pks[j], p.b) && pks[j].t >= 4 && pks[j].t < p.pk_few->t) p.pk_few = &pks[j];
         plan = p;
         return;
       }
@@ -675,6 +687,30 @@ struct Solver {
     if (opt.tile_t > 0 && q.t != opt.tile_t) return false;
     if (opt.threads_kspace > 0 && q.nt != opt.threads_kspace) return false;
     return true;
+  }
+  // The k-space pass of a launch of nb rhs.  Fewer blocks than CUs, or than twice the CUs where a CU holds one
+  // block: the variant with the fewest points a thread (times the rounds its blocks take), the narrower one of
+  // two that are equal: a block's latency is the launch's time (one rhs of 24 x 96 x 160: 18.1 us an iteration with 1024
+  // threads on a 16-wide tile, 21.0 with 256 on an 8-wide one; four of 24 x 216 x 160, 288 blocks of 92 KB or
+  // 576 of 46 KB: 60.4 and 53.9).  Every variant of a split gives the same bits.
+  // Long rows whose neighbouring tiles are on different XCDs (a not a multiple of 8) keep the wide tile:
+  // one rhs of 160 x 80 x 128, a = 20, 33.8 us, 38.7 with an 8-wide tile.
+  const PassKInfo* few_kspace(int nb) const {
+    const auto blocks = [&](int t) { return (long long)nb * plan.a * ((nx + t - 1) / t); };
+    const PassKInfo* best = plan.pk;
+    if (!plan.few_k || (plan.a % 8 != 0 && nx >= 128) || blocks(plan.t) >= (plan.pk->lds > 81920 ? 512 : 256)) return best;
+    const auto cost = [&](const PassKInfo& q) {
+      const long long held = 256ll * std::max(1, std::min(163840 / q.lds, 2048 / q.nt));   // blocks on the chip
+      return (double)((blocks(q.t) + held - 1) / held) * q.t / q.nt;
+    };
+    const PassKInfo* pks = nullptr;
+    const int npk = list_pass_kspace(&pks);
+    for (int j = 0; j < npk; ++j) {
+      if (!fused_ok_k(pks[j], plan.b) || pks[j].t < 4) continue;
+      const double c = cost(pks[j]), cb = cost(*best);
+      if (c < cb || (c == cb && pks[j].t < best->t)) best = &pks[j];
+    }
+    return best;
   }
   std::string shape_str() const {
     return std::to_string(nx) + "x" + std::to_string(ny) + "x" + std::to_string(nz);
@@ -879,10 +915,9 @@ struct Solver {
   // fused schedule for one batch already seeded in fstate
   void run_fused(int nb, int M) {
     const int nv = nb * P;                 // component slots: the real-space pass treats each as an rhs
-    // few blocks: two real-space blocks a CU or less, fewer k-space blocks than CUs (256)
+    // few blocks: two real-space blocks a CU or less
     const PassRInfo* pr = plan.pr_few && (long long)nv * plan.b * nz <= 512 ? plan.pr_few : plan.pr;
-    const PassKInfo* pk =
-        plan.pk_few && (long long)nb * plan.a * ((nx + plan.t - 1) / plan.t) < 256 ? plan.pk_few : plan.pk;
+    const PassKInfo* pk = few_kspace(nb);
     const Consts c = consts(nv);
     const Consts ck = consts(nb);
     const Tables tb = tabs.view();
