@@ -1969,12 +1969,13 @@ struct Solver {
     return best;
   }
 
-  DevBuf<float2> tv_in, tv_y, tv_P;   // used as float arrays for real input
+  DevBuf<float2> tv_in, tv_P;   // used as float arrays for real input
   DevBuf<float2> gr_u, gr_w;
   DevBuf<double2> gr_out;
 
-  // Both element types share the buffers: a real problem of n voxels uses the first
-  // n (or 9n) floats of buffers sized for n complex values.
+  // Both element types share the buffers, which are sized by the problem's own: the input (n values, host data only)
+  // and three dual iterates of 3n values each, a fourth where iterations go two to a launch (real: 36 or 48 bytes
+  // a voxel, complex: 72 or 96).
   void tv_prox(const void* in, void* out, const uint32_t* dims, double lam, double vmin, double vmax,
                double vimag_max, int non_neg, int dirichlet, uint32_t inner, int mem, bool cplx) {
     require(in && out && dims, CBS_ERR_ARG, "null TV argument");
@@ -1984,11 +1985,10 @@ struct Solver {
     const long long n = (long long)dims[0] * dims[1] * dims[2];
     const size_t esz = cplx ? sizeof(float2) : sizeof(float);
     const long long nf = cplx ? 2 * n : n;   // floats per volume
-    tv_y.ensure((size_t)n);
-    tv_P.ensure((size_t)(12 * n));   // P_{k-1}, P_k, P_{k+1} and P_{k+2}
+    auto pairs = [esz](long long values) { return ((size_t)values * esz + sizeof(float2) - 1) / sizeof(float2); };
     const void* din = in;
     if (mem == CBS_MEM_HOST) {
-      tv_in.ensure((size_t)n);
+      tv_in.ensure(pairs(n));
       HIP_CHECK(hipMemcpyAsync(tv_in.p, in, (size_t)n * esz, hipMemcpyHostToDevice, stream));
       din = tv_in.p;
     }
@@ -1997,9 +1997,19 @@ struct Solver {
     a.lam = (float)lam; a.vmin = (float)vmin; a.vmax = (float)vmax;
     a.vimag_max = (vimag_max > 0) ? (float)vimag_max : 0.f;   // NaN or <= 0: no cap (the reference tests > 0)
     a.non_neg = non_neg; a.dirichlet = dirichlet;
+    TvTiles tiles = tv_tiles(a, cplx);
+    if (inner < 3) tiles.gz = 0;   // the first iteration goes alone
+    if (tiles.gz > 0) {
+      try {
+        tv_P.ensure(pairs(12 * n));   // P_{k-1}, P_k, P_{k+1} and P_{k+2}
+      } catch (const CbsError&) {
+        tiles.gz = 0;                 // no room for the fourth: one iteration a launch
+      }
+    }
+    if (tiles.gz == 0) tv_P.ensure(pairs(9 * n));
+    const int np = tiles.gz > 0 ? 4 : 3;
     float* Pk[4];
-    for (int k = 0; k < 4; ++k) Pk[k] = reinterpret_cast<float*>(tv_P.p) + (size_t)k * 3 * nf;
-    float* Y = reinterpret_cast<float*>(tv_y.p);
+    for (int k = 0; k < np; ++k) Pk[k] = reinterpret_cast<float*>(tv_P.p) + (size_t)k * 3 * nf;
     if (inner == 0) hipLaunchKernelGGL(tv_zero, dim3(grid_for(3 * nf)), dim3(256), 0, stream, Pk[0], 3 * nf);
     const unsigned g = grid_for(n);
     int cur = 0, prv = 0;       // P_k in Pk[cur], P_{k-1} in Pk[prv]
@@ -2014,11 +2024,10 @@ struct Solver {
     float theta = 0.f;
     // the first iteration reads no iterate (P_0 = 0); theta is 0 after it, and P_1 stands in for P_0.  The
     // others go two to a launch where that is faster
-    const TvTiles tiles = tv_tiles(a, cplx);
     for (uint32_t it = 0; it < inner;) {
-      // the two buffers that hold neither P_k nor P_{k-1}
-      int nxt[2], m = 0;
-      for (int k = 0; k < 4 && m < 2; ++k)
+      // the buffers that hold neither P_k nor P_{k-1}
+      int nxt[2] = {0, 0}, m = 0;
+      for (int k = 0; k < np && m < 2; ++k)
         if (k != cur && k != prv) nxt[m++] = k;
       if (it > 0 && it + 1 < inner && tiles.gz > 0) {
         const float theta1 = momentum();
@@ -2043,14 +2052,15 @@ struct Solver {
       cur = nxt[0];
       ++it;
     }
-    void* dst = mem == CBS_MEM_HOST ? (void*)Y : out;
+    // the result of host data goes into an iterate that is no longer read
+    void* dst = mem == CBS_MEM_HOST ? (void*)Pk[cur == 0 ? 1 : 0] : out;
     if (cplx)
       hipLaunchKernelGGL(tv_div_project_c, dim3(g), dim3(256), 0, stream, (const float2*)din, (const float2*)Pk[cur],
                          (float2*)dst, a);
     else
       hipLaunchKernelGGL(tv_div_project, dim3(g), dim3(256), 0, stream, (const float*)din, Pk[cur], (float*)dst, a);
     HIP_CHECK(hipGetLastError());
-    if (mem == CBS_MEM_HOST) HIP_CHECK(hipMemcpyAsync(out, Y, (size_t)n * esz, hipMemcpyDeviceToHost, stream));
+    if (mem == CBS_MEM_HOST) HIP_CHECK(hipMemcpyAsync(out, dst, (size_t)n * esz, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
   }
 

@@ -38,3 +38,19 @@ def plane_wave(shape, kx_frac=0.0, ky_frac=0.0, n_m=1.336, wl=0.532, dx=0.1):
 
 def rel(a, b):
     return float(np.linalg.norm(np.ravel(a) - np.ravel(b)) / np.linalg.norm(np.ravel(b)))
+
+
+MB = 1 << 20
+
+
+def take_memory(leave):
+    """Device memory held but for about ``leave`` bytes (a list of tensors: the caller lets go of it)."""
+    import torch
+    hold, size = [], torch.cuda.mem_get_info()[0] - leave
+    while size >= 8 * MB:
+        try:
+            hold.append(torch.empty(size, dtype=torch.uint8, device='cuda'))
+            size = torch.cuda.mem_get_info()[0] - leave
+        except torch.cuda.OutOfMemoryError:
+            size //= 2
+    return hold

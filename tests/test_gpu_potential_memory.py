@@ -3,24 +3,9 @@ that fails, the handle has no potential: solves are refused until the next set_R
 import numpy as np
 import pytest
 
-from helpers import params
+from helpers import MB, params, take_memory
 
 pytestmark = pytest.mark.gpu
-
-MB = 1 << 20
-
-
-def _take_memory(leave):
-    """Device memory held but for about ``leave`` bytes."""
-    import torch
-    hold, size = [], torch.cuda.mem_get_info()[0] - leave
-    while size >= 8 * MB:
-        try:
-            hold.append(torch.empty(size, dtype=torch.uint8, device='cuda'))
-            size = torch.cuda.mem_get_info()[0] - leave
-        except torch.cuda.OutOfMemoryError:
-            size //= 2
-    return hold
 
 
 def test_failed_growth_leaves_no_potential():
@@ -34,7 +19,7 @@ def test_failed_growth_leaves_no_potential():
     s = FORWARD_SOLVER_CONVERGENT_BORN(p)
     s.set_RI(RI + 1j * 1e-3 * (RI > 1.35))
     s.solve_incident(u)                     # the state buffers are there before memory is taken
-    hold = _take_memory(64 * MB)
+    hold = take_memory(64 * MB)
     try:
         if torch.cuda.mem_get_info()[0] > 100 * MB:       # V (262 MB) is given back before the new one is asked for
             pytest.skip('device memory could not be taken')
