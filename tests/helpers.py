@@ -44,13 +44,14 @@ MB = 1 << 20
 
 
 def take_memory(leave):
-    """Device memory held but for about ``leave`` bytes (a list of tensors: the caller lets go of it)."""
-    import torch
-    hold, size = [], torch.cuda.mem_get_info()[0] - leave
+    """Device memory held but for about ``leave`` bytes: a list of buffers, which the caller frees."""
+    from inverse_solver_amd import device as dv
+    hold, size = [], dv.mem_info()[0] - leave
     while size >= 8 * MB:
         try:
-            hold.append(torch.empty(size, dtype=torch.uint8, device='cuda'))
-            size = torch.cuda.mem_get_info()[0] - leave
-        except torch.cuda.OutOfMemoryError:
+            hold.append(dv.DeviceArray((size,), np.uint8))
+            size = dv.mem_info()[0] - leave
+        except RuntimeError:
+            dv.hip.hipGetLastError()        # the refusal is not the next call's error
             size //= 2
     return hold
