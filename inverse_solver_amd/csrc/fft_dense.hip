@@ -505,9 +505,10 @@ __global__ __launch_bounds__(NT) void dense_strided_green3(float2* data, Tables 
 
 // (longest line, threads of the strided kernels, most tasks of a tile).  The strided kernels
 // take 256 threads where four waves hold the tasks: a CU then keeps twice the blocks, and with
-// them twice the waves that have work in the products.
-#define DENSE_LIST(X) X(64, 256, 4) X(64, 512, 8) X(64, 512, 16) X(128, 256, 4) X(128, 512, 8) X(128, 512, 16) \
-  X(192, 512, 8) X(192, 512, 16) X(256, 512, 16) X(320, 512, 16) X(384, 512, 16) X(448, 512, 16) X(448, 512, 32)
+// them twice the waves that have work in the products.  Lines of up to 64 points have at most 4 tasks, of up
+// to 128 at most 8; only 170, 185 and 190 points take (192, 512, 16) and six lengths from 396 on (448, 512, 32).
+#define DENSE_LIST(X) X(64, 256, 4) X(128, 256, 4) X(128, 512, 8) X(192, 512, 8) X(192, 512, 16) X(256, 512, 16) \
+  X(320, 512, 16) X(384, 512, 16) X(448, 512, 16) X(448, 512, 32)
 constexpr int tasks_a_wave(int tasks, int nt) { return (tasks + nt / 64 - 1) / (nt / 64); }
 #define DENSE_ENTRY(N, NT, TASKS)                                                                                  \
   {&dense_rows<N / 64, tasks_a_wave(TASKS, kNT)>, &dense_strided<N * kL / NT, NT, tasks_a_wave(TASKS, NT)>,        \
