@@ -3,7 +3,7 @@ few-block launches: every variant of one split gives the same bits."""
 import numpy as np
 import pytest
 
-from helpers import params, random_field
+from helpers import params, random_field, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +53,16 @@ def test_variants_give_the_same_bits(n, batch):
     got = f.solve_incident(u[..., 0])
     f.close()
     np.testing.assert_array_equal(got, ref[..., 0])
+
+
+# the grids of test_gpu_few_blocks whose single right-hand side runs the batch's own kernels
+@pytest.mark.parametrize('n', [[128, 128, 135], [192, 192, 128], [288, 288, 160]])
+def test_single_rhs_oracle(n):
+    from oracle.cbs import ForwardSolverConvergentBorn as Oracle
+    s, ri, RI = _solver(n, 3)
+    u = random_field(ri, 2)
+    got = s.solve_incident(u)
+    s.close()
+    o = Oracle(params(ri, iterations=3), io_kernels=False, workers=16)
+    o.set_RI(RI)
+    assert rel(got, o.born_loop(u)) < 1e-5
