@@ -1181,7 +1181,7 @@ struct Solver {
     uint64_t b = 3ull * nv * nvox * sizeof(float2);   // field, fstate, spec
     b += 2ull * nv * nri * sizeof(float2);             // staging for host I/O
     b += (uint64_t)nvox * sizeof(float2);   // V
-    if (has_vr()) b += (uint64_t)nvox * sizeof(float);
+    if (v_real) b += (uint64_t)nvox * sizeof(float);   // Vr, in V's allocation whatever the form
     else if (plan.form == CBS_FORM_FUSED) b += (uint64_t)nvox * sizeof(float2);   // its tile-order copy
     b += io.footprint(nv, cx, cy, rz) + (io.ready ? (unsigned long long)nv * nri * 16ull : 0ull);
     return b;

@@ -39,3 +39,23 @@ def test_failed_growth_leaves_no_potential():
     np.testing.assert_array_equal(got, t.solve_incident(u))
     s.close()
     t.close()
+
+
+def test_footprint_counts_the_real_part():
+    """A real RI's potential takes 12 bytes a voxel in every form (complex64 and the real part behind it): the unfused
+    form, which does not read the real part, holds it too."""
+    from inverse_solver_amd import FORWARD_SOLVER_CONVERGENT_BORN
+    ri = (40, 30, 25)
+    p = params(ri, iterations=2)
+    RI = np.full(ri, 1.336)
+    RI[10:20, 10:20, 10:20] = 1.38
+    real, cplx = {}, {}
+    for form in (1, 3):
+        s = FORWARD_SOLVER_CONVERGENT_BORN(p, options=dict(form=form))
+        s.set_RI(RI)
+        real[form] = s.footprint(2)
+        s.set_RI(RI + 1j * 1e-3 * (RI > 1.35))
+        cplx[form] = s.footprint(2)
+        n = int(np.prod(s.simulation_size))
+        s.close()
+    assert real[3] == real[1] == cplx[1] + 4 * n == cplx[3] + 4 * n
