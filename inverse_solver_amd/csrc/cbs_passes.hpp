@@ -772,7 +772,7 @@ __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb
   __shared__ float2 lds[N * T];
   __shared__ float2 s_tw[N];
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(c.nx, N * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks
@@ -827,7 +827,7 @@ __global__ __launch_bounds__(NT) void line_strided_green3(float2* data, Tables t
   __shared__ float2 lds[3 * N * T];
   __shared__ float2 s_tw[N];
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(c.nx, 3 * N * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / T) ny rhs blocks
@@ -913,7 +913,7 @@ __global__ __launch_bounds__(NT) void fft_strided(float2* data, int nx, long lon
   __shared__ float2 s_tw[N];   // twiddles: a task's R1 - 1 of them differ from lane to lane
   for (int i = threadIdx.x; i < N; i += NT) s_tw[i] = tw[i];
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(nx, N * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int tvalid = nx - xt * T < T ? nx - xt * T : T;

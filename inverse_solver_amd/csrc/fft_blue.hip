@@ -115,7 +115,7 @@ __global__ __launch_bounds__(NT) void blue_strided(float2* data, int nx, long lo
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(nx, n * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   if (o >= nouter) return;
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(NT) void blue_strided_green(float2* data, Tables tb
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(c.nx, n * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks

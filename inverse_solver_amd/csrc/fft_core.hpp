@@ -45,13 +45,26 @@ __device__ __forceinline__ void lds_barrier() {
 // Position of block b of nb in an order that gives each of the 8 XCDs (blocks go to them round
 // robin) a contiguous eighth.  For tiles whose rows are not whole 128-byte lines: neighbours
 // write parts of the same lines, which one L2 merges but two pass back and forth, and they read
-// the same lines.  The strided line transforms take it for every row length: 100 x 120 x 75 x 12
-// rhs 7.07 -> 6.02 ms a solve (800-byte rows), 183 x 183 x 83 x 12 73.1 -> 71.6 ms (bound by its
-// arithmetic), 576 x 576 x 320 x 4 543 -> 530 ms (whole lines: neighbouring tiles of a row then
-// share the XCD's translation and memory pages).
+// the same lines: 100 x 120 x 75 x 12 rhs 7.03 -> 6.02 ms a solve (800-byte rows).
 __device__ __forceinline__ unsigned xcd_position(unsigned b, unsigned nb) {
   const unsigned q = nb / 8, r = nb % 8, k = b % 8;
   return k * q + min(k, r) + b / 8;
+}
+// Position of a block of the strided line transforms (tiles of consecutive x of rows of nx, `elems` elements a
+// block).  Rows of whole 128-byte lines have no lines to share.  What the order does there, grouped against plain:
+//  - up to 16 MiB (half the L2s) plain for rows of whole 512 bytes: the blocks in flight then spread over all of a
+//    batch (one rhs of 384 x 50 x 54 47.6 us an iteration grouped, 41.6 plain; of 128 x 98 x 83 54.7, 49.1); other
+//    rows gain 5 to 11 % from 4 rhs on (8 of 48 x 50 x 54 37.2, 41.9);
+//  - from there on within 2 %, but 96 to 256 MiB plain (8 rhs of 256 x 183 x 75 575 and 555, 64 of 160 x 50 x 54
+//    583 and 561);
+//  - above, what the Infinity Cache no longer holds, grouped: neighbouring tiles of a row share the XCD's
+//    translations and memory pages (4 rhs of 256 x 250 x 225 1104 and 1207; 576 x 576 x 320 x 4 530 and 543 ms a solve).
+// (Both orders are formed and one is picked by a mask: a branch holds up the loads of the other arguments, 1 to 2 %.)
+__device__ __forceinline__ unsigned tile_position(int nx, unsigned elems) {
+  const unsigned b = blockIdx.x, nb = gridDim.x;
+  const unsigned size = __umulhi(nb, elems << 12);          // units of 8 MiB (2^20 complex64)
+  const unsigned spread = unsigned((nx & 15) == 0) & (unsigned(size - 12u < 20u) | (unsigned(size < 2) & unsigned((nx & 63) == 0)));
+  return b ^ ((b ^ xcd_position(b, nb)) & (spread - 1u));
 }
 
 // ---------------------------------------------------------------- compile-time trig

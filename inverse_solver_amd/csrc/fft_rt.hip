@@ -154,7 +154,7 @@ __global__ void fft_strided_rt(float2* data, int nx, long long es, long long os,
   float2* a = rt_lds;
   float2* b = rt_lds + (long long)T * L;
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = xcd_position(blockIdx.x, gridDim.x);
+  const unsigned bid = tile_position(nx, p.n * T);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   if (o >= nouter) return;
