@@ -66,8 +66,9 @@ __device__ __forceinline__ void tv_div_project_body(const T* __restrict__ in, co
 // 10 values a voxel, where separate kernels for y and the dual update moved 18 (R read
 // twice and written, y written and read).
 //
-// A block takes a 62 x 6 tile of (x, y) columns, one thread a column and one more each side,
-// and ZC = 3 planes of z.  It requests every operand of its planes before the first is used
+// A block takes a tile of (x, y) columns, 62 x 6 or another shape of its 512 threads on grids that one covers
+// with fewer blocks (tv_columns), one thread a column and one more each side, and ZC = 3 planes of z.  It
+// requests every operand of its planes before the first is used
 // (with one plane requested ahead of the other the launch waited for memory once a plane), then
 // walks up z: the R_x and R_y of the lower neighbours and then the y of the upper ones pass
 // through LDS; R_z and y of the plane below stay in registers.
@@ -81,7 +82,7 @@ __device__ __forceinline__ void tv_div_project_body(const T* __restrict__ in, co
 // FIRST: P_k = P_{k-1} = 0 (no buffer is read, so none has to be cleared).
 // Off: type of a byte offset inside one z plane (32 bits but for planes of 4 GiB and more); the
 // plane's base is uniform, so every access is a scalar base and this offset.
-constexpr int kTvX = 64, kTvY = 8;
+constexpr int kTvT = 512;       // threads: 2^lg columns in x, the rest in y
 
 // 1 / sqrt(s) for s >= 1: the hardware's (1 ulp) and one Newton step; infinity gives 0 and NaN NaN.
 __device__ __forceinline__ float tv_rsqrt(float s) {
@@ -90,26 +91,27 @@ __device__ __forceinline__ float tv_rsqrt(float s) {
   return s < 3.0e38f ? fmaf(0.5f * r, e, r) : r;
 }
 
-template <class T, int ZC, bool FIRST, class Off>
-__global__ __launch_bounds__(kTvX * kTvY) void tv_inner(const T* __restrict__ in, const T* __restrict__ Pc,
-                                                        const T* __restrict__ Pp, T* __restrict__ Pn, TvArgs a,
-                                                        float theta) {
-  __shared__ T sx[kTvY * kTvX], sz[kTvY * kTvX], sy[kTvY * kTvX];   // R_x, R_y and y of a plane
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const unsigned gx = (a.nx + kTvX - 3) / (kTvX - 2), gy = (a.ny + kTvY - 3) / (kTvY - 2);
+// LG: 2^LG threads in x; 0: lg_ at run time (the shifts cost 2 to 12 % of a launch, so the usual shape is compiled).
+template <class T, int ZC, bool FIRST, class Off, int LG>
+__global__ __launch_bounds__(kTvT) void tv_inner(const T* __restrict__ in, const T* __restrict__ Pc,
+                                                 const T* __restrict__ Pp, T* __restrict__ Pn, TvArgs a,
+                                                 float theta, int lg_) {
+  __shared__ T sx[kTvT], sz[kTvT], sy[kTvT];   // R_x, R_y and y of a plane
+  const int lg = LG > 0 ? LG : lg_, nt = 1 << lg, mt = kTvT >> lg;
+  const int tx = threadIdx.x, ty = threadIdx.y, me = ty * nt + tx;
+  const unsigned gx = (a.nx + nt - 3) / (nt - 2), gy = (a.ny + mt - 3) / (mt - 2);
   const unsigned pos = xcd_position(blockIdx.x, gridDim.x), bx = pos % gx, byz = pos / gx;
-  const int x = (int)bx * (kTvX - 2) + tx - 1, y = (int)(byz % gy) * (kTvY - 2) + ty - 1;
+  const int x = (int)bx * (nt - 2) + tx - 1, y = (int)(byz % gy) * (mt - 2) + ty - 1;
   const int z0 = (int)(byz / gy) * ZC, z1 = min(z0 + ZC, a.nz);
-  const bool mine = tx > 0 && tx < kTvX - 1 && ty > 0 && ty < kTvY - 1 && x < a.nx && y < a.ny;
+  const bool mine = tx > 0 && tx < nt - 1 && ty > 0 && ty < mt - 1 && x < a.nx && y < a.ny;
   // periodic column of this thread (columns past the upper neighbour of the last one are not
   // used: they take the last column)
   const int xw = x < 0 ? a.nx - 1 : x < a.nx ? x : x == a.nx ? 0 : a.nx - 1;
   const int yw = y < 0 ? a.ny - 1 : y < a.ny ? y : y == a.ny ? 0 : a.ny - 1;
   const Off col = ((Off)yw * (Off)a.nx + (Off)xw) * (Off)sizeof(T);
   const long long nxy = (long long)a.nx * a.ny, n = nxy * a.nz;
-  const int me = ty * kTvX + tx;
-  const int lx = me - (tx > 0), ly = ty > 0 ? me - kTvX : me;                    // lower neighbours
-  const int ux = me + (tx < kTvX - 1), uy = ty < kTvY - 1 ? me + kTvX : me;      // upper neighbours
+  const int lx = me - (tx > 0), ly = ty > 0 ? me - nt : me;                    // lower neighbours
+  const int ux = me + (tx < nt - 1), uy = ty < mt - 1 ? me + nt : me;          // upper neighbours
   const float c = 1.0f / (12.0f * a.lam);
   const bool edge = a.dirichlet && (xw == 0 || yw == 0 || xw == a.nx - 1 || yw == a.ny - 1);
   auto ld = [&](const T* plane) { return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(plane) + col); };
@@ -332,16 +334,43 @@ __global__ void tv_div_project_c(const float2* __restrict__ in, const float2* __
   tv_div_project_body(in, Q, y, a);
 }
 
+// Columns of a tv_inner block and the blocks of one layer: 64 x 8 threads, or the shape that needs the fewest blocks
+// where that is a third less, counting what short rows cost in memory access (an iteration of 26 x 148 x 44 6.4 -> 5.4
+// us real, 8.4 -> 6.1 complex; 1 x 500 x 500 59 -> 7 us; but 64 x 64 x 65 real with 32 threads in x, 15 for 22 blocks,
+// 5.9 -> 6.4, and 83 x 62 x 45 with 8 6.0 -> 7.4).
+struct TvColumns {
+  int lg;                   // 2^lg threads in x
+  unsigned gx, gy;
+};
+static TvColumns tv_columns(const TvArgs& a) {
+  auto of = [&](int lg) {
+    const unsigned nt = 1u << lg, mt = (unsigned)kTvT >> lg;
+    return TvColumns{lg, (a.nx + nt - 3) / (nt - 2), (a.ny + mt - 3) / (mt - 2)};
+  };
+  auto cost = [](const TvColumns& c) {
+    const double row[] = {0, 0, 2.0, 1.5, 1.15, 1.0, 1.0, 1.0};
+    return (double)c.gx * c.gy * row[c.lg];
+  };
+  TvColumns best = of(6);
+  const double limit = 0.65 * cost(best);
+  for (int lg : {7, 5, 4, 3, 2}) {
+    const TvColumns c = of(lg);
+    if (cost(c) <= limit && cost(c) < cost(best)) best = c;
+  }
+  return best;
+}
+constexpr int kTvZ = 3;
+
 template <class T, class Off>
 static void launch_inner(hipStream_t st, const T* in, const T* Pc, const T* Pp, T* Pn, const TvArgs& a, float theta,
                          bool first) {
-  constexpr int ZC = 3;
-  const unsigned gx = (unsigned)((a.nx + kTvX - 3) / (kTvX - 2)), gy = (unsigned)((a.ny + kTvY - 3) / (kTvY - 2));
-  const dim3 grid(gx * gy * (unsigned)((a.nz + ZC - 1) / ZC)), block(kTvX, kTvY);
-  if (first)
-    hipLaunchKernelGGL((tv_inner<T, ZC, true, Off>), grid, block, 0, st, in, Pc, Pp, Pn, a, theta);
-  else
-    hipLaunchKernelGGL((tv_inner<T, ZC, false, Off>), grid, block, 0, st, in, Pc, Pp, Pn, a, theta);
+  const TvColumns c = tv_columns(a);
+  const dim3 grid(c.gx * c.gy * (unsigned)((a.nz + kTvZ - 1) / kTvZ)), block(1u << c.lg, (unsigned)kTvT >> c.lg);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, in, Pc, Pp, Pn, a, theta, c.lg); };
+  if (c.lg == 6 && first) launch(tv_inner<T, kTvZ, true, Off, 6>);
+  else if (c.lg == 6) launch(tv_inner<T, kTvZ, false, Off, 6>);
+  else if (first) launch(tv_inner<T, kTvZ, true, Off, 0>);
+  else launch(tv_inner<T, kTvZ, false, Off, 0>);
 }
 template <class T>
 static void launch_inner(hipStream_t st, const T* in, const T* Pc, const T* Pp, T* Pn, const TvArgs& a, float theta,
@@ -361,10 +390,12 @@ void tv_inner_complex(hipStream_t st, const float2* in, const float2* Pc, const 
 }
 
 // Tiles of tv_inner2 and whether it pays (gz > 0): columns of up to 60 in x and what the threads of a block
-// hold in y, shared out evenly, and the planes a block that take the least time.  Times in us, fitted to the
-// sizes above and to small ones: a launch of tv_inner2 3 and 1.2 a step (real, one block a CU), 1.75 (two
-// blocks) or 1.8 (complex); two launches of tv_inner 3.3 each and their bytes at 5.2 TB/s, 5.4 at least.
-// 60 x 70 x 40 complex keeps tv_inner (6.8 us an iteration; 7.4), real takes tv_inner2 (5.5; 5.4).
+// hold in y, shared out evenly, and the planes a block that take the least time.  Times in us, fitted to 100 grids from
+// 8^3 to 200 x 190 x 110: a launch of tv_inner2 3 and, a step, what grows with the waves w of a CU, 0.65 + 0.046 w real
+// (24 waves at most: two full blocks) or 0.7 + 0.079 w complex (12); an iteration of tv_inner 3.3 and its bytes at 5.2 TB/s
+// or 3.2 for every three or four blocks of a CU, 5.2 (real) and 6.5 (complex) at least.
+// Small complex grids gain as real ones do (8^3 6.0 -> 3.3 us, 30 x 58 x 119 8.4 -> 6.1); flat ones keep tv_inner
+// (500 x 500 x 1 real 5.5, 7.0; complex 7.0, 12.6).
 TvTiles tv_tiles(const TvArgs& a, bool cplx) {
   TvTiles g;
   g.gx = (a.nx + 59) / 60;
@@ -373,19 +404,26 @@ TvTiles tv_tiles(const TvArgs& a, bool cplx) {
   g.gy = (a.ny + uy - 1) / uy;
   g.ty = (a.ny + g.gy - 1) / g.gy + 4;
   const long long cols = (long long)g.gx * g.gy, cus = 256;
+  const int waves = (g.tx * g.ty + 63) / 64;       // of a block
+  // blocks on a CU: by registers, and by the 18 and 36 KB of LDS
+  const long long held = std::max(1, std::min((cplx ? 12 : 24) / waves, cplx ? 4 : 8));
   double best = 0.0;
   for (int zc = 1; zc <= a.nz; ++zc) {
     const long long nb = cols * ((a.nz + zc - 1) / zc);
-    const bool two = !cplx && nb > cus;            // two blocks a CU
-    const long long rounds = two ? (nb + 2 * cus - 1) / (2 * cus) : (nb + cus - 1) / cus;
-    const double t = 3.0 + (double)rounds * (zc + 4) * (cplx ? 1.8 : two ? 1.75 : 1.2);
-    if (best > 0.0 && t >= best) continue;
-    best = t;
-    g.zc = zc;
+    const long long rounds = (nb + held * cus - 1) / (held * cus);
+    const double w = (double)waves * std::min(held, (nb + cus - 1) / cus);
+    const double t = 3.0 + (double)rounds * (zc + 4) * (cplx ? 0.7 + 0.079 * w : 0.65 + 0.046 * w);
+    if (best == 0.0 || t < best) {
+      best = t;
+      g.zc = zc;
+    }
+    if (nb <= cus) break;                          // one block a CU: more planes a block only take longer
   }
   g.gz = (a.nz + g.zc - 1) / g.zc;
   const double bytes = 10.0 * (cplx ? 8.0 : 4.0) * a.nx * a.ny * a.nz;
-  if (best >= 2.0 * std::max(5.4, 3.3 + bytes / 5.2e6) || cols * g.gz >= (1ll << 31)) g.gz = 0;
+  const TvColumns c = tv_columns(a);
+  const double rounds1 = (double)c.gx * c.gy * ((a.nz + kTvZ - 1) / kTvZ) / (cplx ? 768 : 1024);
+  if (best >= 2.0 * std::max(cplx ? 6.5 : 5.2, 3.3 + std::max(bytes / 5.2e6, 3.2 * rounds1)) || cols * g.gz >= (1ll << 31)) g.gz = 0;
   return g;
 }
 template <class T>
