@@ -44,14 +44,18 @@ MB = 1 << 20
 
 
 def take_memory(leave):
-    """Device memory held but for about ``leave`` bytes: a list of buffers, which the caller frees."""
+    """Device memory held but for ``leave`` bytes and a few MB: a list of buffers, which the caller frees."""
+    import gc
     from inverse_solver_amd import device as dv
-    hold, size = [], dv.mem_info()[0] - leave
-    while size >= 8 * MB:
+    gc.collect()                            # handles of earlier tests would give memory back meanwhile
+    rest = dv.DeviceArray((leave,), np.uint8)
+    # until allocations are refused: the runtime keeps freed memory that it reports as taken
+    hold, size = [], dv.mem_info()[0]
+    while size >= 2 * MB:
         try:
             hold.append(dv.DeviceArray((size,), np.uint8))
-            size = dv.mem_info()[0] - leave
         except RuntimeError:
             dv.hip.hipGetLastError()        # the refusal is not the next call's error
             size //= 2
+    rest.free()
     return hold
