@@ -59,12 +59,20 @@ __device__ __forceinline__ unsigned xcd_position(unsigned b, unsigned nb) {
 //    583 and 561);
 //  - above, what the Infinity Cache no longer holds, grouped: neighbouring tiles of a row share the XCD's
 //    translations and memory pages (4 rhs of 256 x 250 x 225 1104 and 1207; 576 x 576 x 320 x 4 530 and 543 ms a solve).
-// (Both orders are formed and one is picked by a mask: a branch holds up the loads of the other arguments, 1 to 2 %.)
-__device__ __forceinline__ unsigned tile_position(int nx, unsigned elems) {
-  const unsigned b = blockIdx.x, nb = gridDim.x;
-  const unsigned size = __umulhi(nb, elems << 12);          // units of 8 MiB (2^20 complex64)
+// tile_mask: all ones for the grouped order.  Both orders are formed and one is picked by the mask: a branch holds up
+// the loads of the other arguments, 1 to 2 %.  Kernels whose elems is known at compile time form the mask themselves;
+// the matrix-core ones get it from the host (formed there, 183 x 183 x 83 x 12 took 0.7 % longer).
+__host__ __device__ inline unsigned tile_mask(int nx, unsigned nb, unsigned elems) {
+  const unsigned size = (unsigned)(((unsigned long long)nb * (elems << 12)) >> 32);   // units of 8 MiB (2^20 complex64)
   const unsigned spread = unsigned((nx & 15) == 0) & (unsigned(size - 12u < 20u) | (unsigned(size < 2) & unsigned((nx & 63) == 0)));
-  return b ^ ((b ^ xcd_position(b, nb)) & (spread - 1u));
+  return spread - 1u;
+}
+__device__ __forceinline__ unsigned tile_position(unsigned mask) {
+  const unsigned b = blockIdx.x;
+  return b ^ ((b ^ xcd_position(b, gridDim.x)) & mask);
+}
+__device__ __forceinline__ unsigned tile_position(int nx, unsigned elems) {
+  return tile_position(tile_mask(nx, gridDim.x, elems));
 }
 
 // ---------------------------------------------------------------- compile-time trig

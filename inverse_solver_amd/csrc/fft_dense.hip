@@ -394,7 +394,7 @@ __global__ __launch_bounds__(NT) void dense_strided(float2* data, int nx, long l
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x;
   const int ntile = (nx + kL - 1) / kL;
-  const unsigned bid = tile_position(nx, n * kL);
+  const unsigned bid = tile_position(p.grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int tv = nx - xt * kL < kL ? nx - xt * kL : kL;
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(NT) void dense_strided_green(float2* data, Tables t
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x;
   const int ntile = (c.nx + kL - 1) / kL;
-  const unsigned bid = tile_position(c.nx, n * kL);
+  const unsigned bid = tile_position(p.grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / 16) ny slots blocks
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(NT) void dense_strided_green3(float2* data, Tables 
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x, tile = n * kL;
   const int ntile = (c.nx + kL - 1) / kL;
-  const unsigned bid = tile_position(c.nx, 3 * n * kL);
+  const unsigned bid = tile_position(p.grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / 16) ny rhs blocks

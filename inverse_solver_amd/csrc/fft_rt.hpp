@@ -64,6 +64,7 @@ struct DenseArgs {
   int inv_F;                // ceil(65536 / F): task / F = task inv_F >> 16
   float inv_m;              // 1 / m
   const float2* tab;        // [m] (cos, sin)(2 pi e / m), then [n] exp(-2 pi i e / n)
+  unsigned grouped;         // strided launches: tile_mask of the launch
 };
 // values of the tables a block holds
 __host__ __device__ inline int dense_tables(const DenseArgs& a) { return a.m + (a.F > 1 ? a.n : 0); }
@@ -82,6 +83,11 @@ struct DenseInfo {
   // dynamic LDS: the tables and the tile (rows: one word of padding an element)
   size_t lds_rows(const DenseArgs& a) const { return (size_t)(a.n * (lines + 1) + dense_tables(a)) * sizeof(float2); }
   size_t lds_strided(const DenseArgs& a) const { return (size_t)(a.n * lines + dense_tables(a)) * sizeof(float2); }
+  // a strided launch of nb blocks over rows of nx, comps components a block
+  DenseArgs strided_args(DenseArgs a, int nx, long long nb, int comps) const {
+    a.grouped = tile_mask(nx, (unsigned)nb, (unsigned)(comps * a.n * lines));
+    return a;
+  }
   size_t lds_green3(const DenseArgs& a) const { return lds_strided(a) + (size_t)(2 * a.n * lines) * sizeof(float2); }
 };
 // the kernels for lines of n elements and ntask tasks (null: too long)

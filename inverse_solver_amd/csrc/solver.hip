@@ -450,8 +450,8 @@ struct Solver {
       const long long nblk = (long long)((ncols + P.di->lines - 1) / P.di->lines) * nouter;
       require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
       timed(2, [&] { hipLaunchKernelGGL(P.di->strided, dim3((unsigned)nblk), dim3(P.di->nt_strided),
-                                        P.di->lds_strided(P.da), stream, data, ncols, es, os, (int)nouter, P.da,
-                                        inverse, in, os2); });
+                                        P.di->lds_strided(P.da), stream, data, ncols, es, os, (int)nouter,
+                                        P.di->strided_args(P.da, ncols, nblk, 1), inverse, in, os2); });
       return;
     }
     if (P.bi) {
@@ -1123,8 +1123,8 @@ struct Solver {
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
         const size_t lds = P == 3 ? dz->lds_green3(rtp[2].da) : dz->lds_strided(rtp[2].da);
         timed(2, [&] { hipLaunchKernelGGL(P == 3 ? dz->strided_green3 : dz->strided_green, dim3((unsigned)nblk),
-                                          dim3(dz->nt_strided), lds, stream, ws.spec, tb, c, rtp[2].da, ws.parity, jj,
-                                          cv); });
+                                          dim3(dz->nt_strided), lds, stream, ws.spec, tb, c,
+                                          dz->strided_args(rtp[2].da, nx, nblk, P), ws.parity, jj, cv); });
         return;
       }
       if (!bz) {
