@@ -819,7 +819,7 @@ __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb
 // The same for vector runs: a block holds the three components of its lines (component q's line l at index
 // q T + l of a row of the tile) and applies the dyadic factor of green_plain_vec between the transforms, where
 // the transforms and the factor on their own moved each component three times.  With the x passes fused as well,
-// 100 x 120 x 75 x 4 rhs of three components went from 375 to 200 us an iteration.
+// 100 x 120 x 75 x 4 rhs of three components went from 372 to 196 us an iteration.
 template <int N, int T, int NT>
 __global__ __launch_bounds__(NT) void line_strided_green3(float2* data, Tables tb, Consts c, const float2* tw,
                                                           const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {

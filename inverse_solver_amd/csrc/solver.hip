@@ -1811,7 +1811,8 @@ struct Solver {
     if (prm.acyclic) flip_state = (int)((flip_state + (long long)n_rhs * M) & 1);
   }
 
-  // Times every fused plan for the grid and keeps the fastest.
+  // Times every fused plan for the grid and keeps the fastest, which then runs at every batch width (the options
+  // hold its tile and threads, so launches of few blocks take no other variants).
   double autotune(uint32_t n_rhs, uint32_t iters) {
     require(have_potential, CBS_ERR_STATE, "cbs_set_potential must be called before cbs_autotune");
     require(n_rhs >= 1 && iters >= 3, CBS_ERR_ARG, "autotune needs n_rhs >= 1 and iterations >= 3");
