@@ -767,12 +767,13 @@ __global__ __launch_bounds__(NT) void line_rows_update(StateArgs st, Tables tb, 
 // Tiles as fft_strided: T consecutive x positions of z lines, outer set o = y + ny slot.
 template <int N, int T, int NT>
 __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb, Consts c, const float2* tw,
-                                                         const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+                                                         const uint8_t* __restrict__ parity, int jj, ConvArgs cv,
+                                                         unsigned grouped) {
   constexpr int K = (N * T + NT - 1) / NT;
   __shared__ float2 lds[N * T];
   __shared__ float2 s_tw[N];
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = tile_position(c.nx, N * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks
@@ -822,12 +823,13 @@ __global__ __launch_bounds__(NT) void line_strided_green(float2* data, Tables tb
 // 100 x 120 x 75 x 4 rhs of three components went from 372 to 196 us an iteration.
 template <int N, int T, int NT>
 __global__ __launch_bounds__(NT) void line_strided_green3(float2* data, Tables tb, Consts c, const float2* tw,
-                                                          const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+                                                          const uint8_t* __restrict__ parity, int jj, ConvArgs cv,
+                                                          unsigned grouped) {
   constexpr int K = (N * T + NT - 1) / NT;
   __shared__ float2 lds[3 * N * T];
   __shared__ float2 s_tw[N];
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = tile_position(c.nx, 3 * N * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / T) ny rhs blocks
@@ -908,12 +910,13 @@ __global__ __launch_bounds__(NT) void fft_rows(float2* data, long long nrows, co
 // y positions of a z transform and the right-hand sides).
 template <int N, int T, int NT>
 __global__ __launch_bounds__(NT) void fft_strided(float2* data, int nx, long long es, long long os, int nouter,
-                                                  const float2* tw, int inverse, int inner, long long os2) {
+                                                  const float2* tw, int inverse, int inner, long long os2,
+                                                  unsigned grouped) {
   __shared__ float2 lds[N * T];
   __shared__ float2 s_tw[N];   // twiddles: a task's R1 - 1 of them differ from lane to lane
   for (int i = threadIdx.x; i < N; i += NT) s_tw[i] = tw[i];
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = tile_position(nx, N * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int tvalid = nx - xt * T < T ? nx - xt * T : T;

@@ -106,7 +106,8 @@ __global__ __launch_bounds__(NT) void blue_rows(float2* data, long long nrows, B
 // base = (o / inner) os2 + (o % inner) os + xt T.  Loads issued as in blue_rows.
 template <int L, int T, int NT>
 __global__ __launch_bounds__(NT) void blue_strided(float2* data, int nx, long long es, long long os, int nouter,
-                                                   BlueArgs p, int inverse, int inner, long long os2) {
+                                                   BlueArgs p, int inverse, int inner, long long os2,
+                                                   unsigned grouped) {
   constexpr int NMAX = (L + 1) / 2;
   constexpr int K = (NMAX * T + NT - 1) / NT;
   constexpr int KZ = ((L - NMAX) * T + NT - 1) / NT;
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(NT) void blue_strided(float2* data, int nx, long lo
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = tile_position(nx, n * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   if (o >= nouter) return;
@@ -296,7 +297,8 @@ __global__ __launch_bounds__(NT) void blue_rows_update(StateArgs st, Tables tb, 
 // one launch.  Tiles as blue_strided with es = nx ny and outer set o = y + ny slot.
 template <int L, int T, int NT>
 __global__ __launch_bounds__(NT) void blue_strided_green(float2* data, Tables tb, Consts c, BlueArgs p,
-                                                         const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+                                                         const uint8_t* __restrict__ parity, int jj, ConvArgs cv,
+                                                         unsigned grouped) {
   constexpr int NMAX = (L + 1) / 2;
   constexpr int K = (NMAX * T + NT - 1) / NT;
   constexpr int KZ = ((L - NMAX) * T + NT - 1) / NT;
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(NT) void blue_strided_green(float2* data, Tables tb
   __shared__ float2 s_b[L];
   const int n = p.n;
   const int ntile = (c.nx + T - 1) / T;
-  const unsigned bid = tile_position(c.nx, n * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / T) ny slots blocks

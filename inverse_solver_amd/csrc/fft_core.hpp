@@ -51,7 +51,7 @@ __device__ __forceinline__ unsigned xcd_position(unsigned b, unsigned nb) {
   return k * q + min(k, r) + b / 8;
 }
 // Position of a block of the strided line transforms (tiles of consecutive x of rows of nx, `elems` elements a
-// block).  Rows of whole 128-byte lines have no lines to share.  What the order does there, grouped against plain:
+// block, nb blocks).  Rows of whole 128-byte lines have no lines to share.  What the order does there, grouped against plain:
 //  - up to 16 MiB (half the L2s) plain for rows of whole 512 bytes: the blocks in flight then spread over all of a
 //    batch (one rhs of 384 x 50 x 54 47.6 us an iteration grouped, 41.6 plain; of 128 x 98 x 83 54.7, 49.1); other
 //    rows gain 5 to 11 % from 4 rhs on (8 of 48 x 50 x 54 37.2, 41.9);
@@ -59,20 +59,17 @@ __device__ __forceinline__ unsigned xcd_position(unsigned b, unsigned nb) {
 //    583 and 561);
 //  - above, what the Infinity Cache no longer holds, grouped: neighbouring tiles of a row share the XCD's
 //    translations and memory pages (4 rhs of 256 x 250 x 225 1104 and 1207; 576 x 576 x 320 x 4 530 and 543 ms a solve).
-// tile_mask: all ones for the grouped order.  Both orders are formed and one is picked by the mask: a branch holds up
-// the loads of the other arguments, 1 to 2 %.  Kernels whose elems is known at compile time form the mask themselves;
-// the matrix-core ones get it from the host (formed there, 183 x 183 x 83 x 12 took 0.7 % longer).
-__host__ __device__ inline unsigned tile_mask(int nx, unsigned nb, unsigned elems) {
-  const unsigned size = (unsigned)(((unsigned long long)nb * (elems << 12)) >> 32);   // units of 8 MiB (2^20 complex64)
-  const unsigned spread = unsigned((nx & 15) == 0) & (unsigned(size - 12u < 20u) | (unsigned(size < 2) & unsigned((nx & 63) == 0)));
-  return spread - 1u;
+// tile_mask (host): the launch's last argument, all ones for the grouped order.  Both orders are formed and one is
+// picked by the mask: a branch holds up the loads of the other arguments, 1 to 2 %; formed in the kernels the mask
+// cost 0.3 (100 x 120 x 75 x 12) to 0.7 % (183 x 183 x 83 x 12).
+inline unsigned tile_mask(int nx, long long nb, int elems) {
+  const long long size = nb * elems >> 20;                  // units of 8 MiB
+  const bool spread = nx % 16 == 0 && ((size >= 12 && size < 32) || (size < 2 && nx % 64 == 0));
+  return spread ? 0u : ~0u;
 }
-__device__ __forceinline__ unsigned tile_position(unsigned mask) {
+__device__ __forceinline__ unsigned tile_position(unsigned grouped) {
   const unsigned b = blockIdx.x;
-  return b ^ ((b ^ xcd_position(b, gridDim.x)) & mask);
-}
-__device__ __forceinline__ unsigned tile_position(int nx, unsigned elems) {
-  return tile_position(tile_mask(nx, gridDim.x, elems));
+  return b ^ ((b ^ xcd_position(b, gridDim.x)) & grouped);
 }
 
 // ---------------------------------------------------------------- compile-time trig

@@ -389,12 +389,12 @@ __device__ __forceinline__ void store_strided(float2* __restrict__ base, long lo
 
 template <int KC, int NT, int TPW>
 __global__ __launch_bounds__(NT) void dense_strided(float2* data, int nx, long long es, long long os, int nouter,
-                                                     DenseArgs p, int inverse, int inner, long long os2) {
+                                                     DenseArgs p, int inverse, int inner, long long os2, unsigned grouped) {
   extern __shared__ float2 s_tw[];
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x;
   const int ntile = (nx + kL - 1) / kL;
-  const unsigned bid = tile_position(p.grouped);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int tv = nx - xt * kL < kL ? nx - xt * kL : kL;
@@ -415,12 +415,13 @@ __global__ __launch_bounds__(NT) void dense_strided(float2* data, int nx, long l
 // green_plain and the inverse z transform in one launch.
 template <int KC, int NT, int TPW>
 __global__ __launch_bounds__(NT) void dense_strided_green(float2* data, Tables tb, Consts c, DenseArgs p,
-                                                           const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+                                                           const uint8_t* __restrict__ parity, int jj, ConvArgs cv,
+                                                           unsigned grouped) {
   extern __shared__ float2 s_tw[];
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x;
   const int ntile = (c.nx + kL - 1) / kL;
-  const unsigned bid = tile_position(p.grouped);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, slot = o / c.ny;      // the grid holds ceil(nx / 16) ny slots blocks
@@ -460,12 +461,13 @@ __global__ __launch_bounds__(NT) void dense_strided_green(float2* data, Tables t
 // iteration (Bluestein's transforms and separate passes before).
 template <int KC, int NT, int TPW>
 __global__ __launch_bounds__(NT) void dense_strided_green3(float2* data, Tables tb, Consts c, DenseArgs p,
-                                                            const uint8_t* __restrict__ parity, int jj, ConvArgs cv) {
+                                                            const uint8_t* __restrict__ parity, int jj, ConvArgs cv,
+                                                           unsigned grouped) {
   extern __shared__ float2 s_tw[];
   float2* lds = s_tw + dense_tables(p);
   const int n = p.n, tid = threadIdx.x, tile = n * kL;
   const int ntile = (c.nx + kL - 1) / kL;
-  const unsigned bid = tile_position(p.grouped);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   const int y = o % c.ny, r = o / c.ny;         // the grid holds ceil(nx / 16) ny rhs blocks

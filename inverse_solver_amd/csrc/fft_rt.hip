@@ -148,13 +148,13 @@ __global__ void fft_rows_rt(float2* data, long long nrows, RtFft p, int lines_pe
 }
 
 __global__ void fft_strided_rt(float2* data, int nx, long long es, long long os, int nouter, RtFft p, int T,
-                               int inverse, int inner, long long os2) {
+                               int inverse, int inner, long long os2, unsigned grouped) {
   extern __shared__ float2 rt_lds[];
   const int L = p.L, n = p.n;
   float2* a = rt_lds;
   float2* b = rt_lds + (long long)T * L;
   const int ntile = (nx + T - 1) / T;
-  const unsigned bid = tile_position(nx, p.n * T);
+  const unsigned bid = tile_position(grouped);
   const int xt = bid % ntile;
   const int o = bid / ntile;
   if (o >= nouter) return;

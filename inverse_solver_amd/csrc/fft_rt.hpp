@@ -43,7 +43,7 @@ __global__ void fft_rows_rt(float2* data, long long nrows, RtFft p, int lines_pe
 // base = (o / inner) * os2 + (o % inner) * os + xt * T.  T = rt_lines(p.L, 16); dynamic
 // LDS = 2 * T * p.L * 8 bytes.
 __global__ void fft_strided_rt(float2* data, int nx, long long es, long long os, int nouter, RtFft p, int T,
-                               int inverse, int inner, long long os2);
+                               int inverse, int inner, long long os2, unsigned grouped);
 
 // Bluestein's transform on a compiled convolution length L >= 2n - 1 (fft_blue.hip):
 // the chirp products are fused into the tile load and store, and the convolution is
@@ -64,14 +64,13 @@ struct DenseArgs {
   int inv_F;                // ceil(65536 / F): task / F = task inv_F >> 16
   float inv_m;              // 1 / m
   const float2* tab;        // [m] (cos, sin)(2 pi e / m), then [n] exp(-2 pi i e / n)
-  unsigned grouped;         // strided launches: tile_mask of the launch
 };
 // values of the tables a block holds
 __host__ __device__ inline int dense_tables(const DenseArgs& a) { return a.m + (a.F > 1 ? a.n : 0); }
 using DenseRowsFn = void (*)(float2*, long long, DenseArgs, int);
-using DenseStridedFn = void (*)(float2*, int, long long, long long, int, DenseArgs, int, int, long long);
+using DenseStridedFn = void (*)(float2*, int, long long, long long, int, DenseArgs, int, int, long long, unsigned);
 using DenseRowsUpdateFn = void (*)(StateArgs, Tables, Consts, DenseArgs, int, int, int, int, ConvArgs);
-using DenseStridedGreenFn = void (*)(float2*, Tables, Consts, DenseArgs, const uint8_t*, int, ConvArgs);
+using DenseStridedGreenFn = void (*)(float2*, Tables, Consts, DenseArgs, const uint8_t*, int, ConvArgs, unsigned);
 struct DenseInfo {
   DenseRowsFn rows;
   DenseStridedFn strided;
@@ -83,11 +82,6 @@ struct DenseInfo {
   // dynamic LDS: the tables and the tile (rows: one word of padding an element)
   size_t lds_rows(const DenseArgs& a) const { return (size_t)(a.n * (lines + 1) + dense_tables(a)) * sizeof(float2); }
   size_t lds_strided(const DenseArgs& a) const { return (size_t)(a.n * lines + dense_tables(a)) * sizeof(float2); }
-  // a strided launch of nb blocks over rows of nx, comps components a block
-  DenseArgs strided_args(DenseArgs a, int nx, long long nb, int comps) const {
-    a.grouped = tile_mask(nx, (unsigned)nb, (unsigned)(comps * a.n * lines));
-    return a;
-  }
   size_t lds_green3(const DenseArgs& a) const { return lds_strided(a) + (size_t)(2 * a.n * lines) * sizeof(float2); }
 };
 // the kernels for lines of n elements and ntask tasks (null: too long)
@@ -95,11 +89,11 @@ const DenseInfo* find_dense(int n, int ntask);
 
 // rows: NL contiguous lines of n per block; strided: as fft_strided_rt with T = t lines
 using BlueRowsFn = void (*)(float2*, long long, BlueArgs, int);
-using BlueStridedFn = void (*)(float2*, int, long long, long long, int, BlueArgs, int, int, long long);
+using BlueStridedFn = void (*)(float2*, int, long long, long long, int, BlueArgs, int, int, long long, unsigned);
 // per-axis form, one field component: x inverse + pointwise update + x forward, and z
 // forward + Green's multiply + z inverse (fft_blue.hip)
 using BlueRowsUpdateFn = void (*)(StateArgs, Tables, Consts, BlueArgs, int, int, int, int, ConvArgs);
-using BlueStridedGreenFn = void (*)(float2*, Tables, Consts, BlueArgs, const uint8_t*, int, ConvArgs);
+using BlueStridedGreenFn = void (*)(float2*, Tables, Consts, BlueArgs, const uint8_t*, int, ConvArgs, unsigned);
 struct BlueInfo {
   BlueRowsFn rows;
   BlueStridedFn strided;

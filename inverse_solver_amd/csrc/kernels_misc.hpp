@@ -40,7 +40,7 @@ __global__ void potential_fill(RiGrid g, int flip_conj, RoiGeom rg, int snx, int
 using PassRFn = void (*)(struct PassRArgs);
 using PassKFn = void (*)(struct PassKArgs);
 using RowsFn = void (*)(float2*, long long, const float2*, int);
-using StridedFn = void (*)(float2*, int, long long, long long, int, const float2*, int, int, long long);
+using StridedFn = void (*)(float2*, int, long long, long long, int, const float2*, int, int, long long, unsigned);
 
 // fn takes every update kind; fn_steady only UPD_DEFER / UPD_PAIR with FWD_GAMMA
 // fn_vr, fn_steady_vr: the same passes reading a real potential (st.Vr)
@@ -56,7 +56,7 @@ const StridedInfo* find_fft_strided(int n, int t);
 // per-axis form, one field component, compiled line lengths (lines_fused_inst.hip):
 // x inverse + pointwise update + x forward, and z forward + Green's multiply + z inverse
 using RowsUpdateFn = void (*)(StateArgs, Tables, Consts, const float2*, int, int, int, int, ConvArgs);
-using StridedGreenFn = void (*)(float2*, Tables, Consts, const float2*, const uint8_t*, int, ConvArgs);
+using StridedGreenFn = void (*)(float2*, Tables, Consts, const float2*, const uint8_t*, int, ConvArgs, unsigned);
 struct RowsUpdateInfo { RowsUpdateFn fn, fn_vr; int n, rows, nt; };   // fn_vr: real potential (st.Vr)
 struct StridedGreenInfo { StridedGreenFn fn; int n, t, nt; };
 const RowsUpdateInfo* find_rows_update(int n);

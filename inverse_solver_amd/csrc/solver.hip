@@ -451,7 +451,7 @@ struct Solver {
       require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
       timed(2, [&] { hipLaunchKernelGGL(P.di->strided, dim3((unsigned)nblk), dim3(P.di->nt_strided),
                                         P.di->lds_strided(P.da), stream, data, ncols, es, os, (int)nouter,
-                                        P.di->strided_args(P.da, ncols, nblk, 1), inverse, in, os2); });
+                                        P.da, inverse, in, os2, tile_mask(ncols, nblk, P.da.n * P.di->lines)); });
       return;
     }
     if (P.bi) {
@@ -459,7 +459,7 @@ struct Solver {
       const long long nblk = (long long)((ncols + T - 1) / T) * nouter;
       require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
       timed(2, [&] { hipLaunchKernelGGL(P.bi->strided, dim3((unsigned)nblk), dim3(P.bi->nt), 0, stream, data, ncols,
-                                        es, os, (int)nouter, P.ba, inverse, in, os2); });
+                                        es, os, (int)nouter, P.ba, inverse, in, os2, tile_mask(ncols, nblk, P.k.n * T)); });
       return;
     }
     const int T = rt_lines(P.k.L, 16);
@@ -467,7 +467,7 @@ struct Solver {
     require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "run-time FFT batch too large for one launch");
     const size_t lds = 2ull * T * P.k.L * sizeof(float2);
     timed(2, [&] { hipLaunchKernelGGL(fft_strided_rt, dim3((unsigned)nblk), dim3(256), lds, stream, data, ncols,
-                                      es, os, (int)nouter, P.k, T, inverse, in, os2); });
+                                      es, os, (int)nouter, P.k, T, inverse, in, os2, tile_mask(ncols, nblk, P.k.n * T)); });
   }
 
   void drop_graph() {
@@ -1003,7 +1003,8 @@ struct Solver {
       const long long nouter = (long long)nz * nv;
       const dim3 g((unsigned)(nt * nouter));
       timed(2, [&] { hipLaunchKernelGGL(sy->fn, g, dim3(sy->nt), 0, stream, ws.spec, nx, (long long)nx,
-                                        (long long)nx * ny, (int)nouter, tabs.tw_y.p, inverse, (int)nouter, 0ll); });
+                                        (long long)nx * ny, (int)nouter, tabs.tw_y.p, inverse, (int)nouter, 0ll,
+                                        tile_mask(nx, nt * nouter, sy->n * sy->t)); });
     };
     pass_r(UPD_NONE, FWD_P0, 0, 1);
     for (int jj = 1; jj <= M; ++jj) {
@@ -1053,7 +1054,7 @@ struct Solver {
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "y transform batch too large for one launch");
         timed(2, [&] { hipLaunchKernelGGL(sy->fn, dim3((unsigned)nblk), dim3(sy->nt), 0, stream, sp, nx,
                                           (long long)nx, (long long)nx * ny, (int)nouter, tabs.tw_a.p, inverse,
-                                          (int)nouter, 0ll); });
+                                          (int)nouter, 0ll, tile_mask(nx, nblk, sy->n * sy->t)); });
       };
       auto fz = [&] {   // outer: y (nx apart) within a slot, then the slots (nvox apart)
         const long long nouter = (long long)ny * nv;
@@ -1063,7 +1064,7 @@ struct Solver {
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
         timed(2, [&] { hipLaunchKernelGGL(sz->fn, dim3((unsigned)nblk), dim3(sz->nt), 0, stream, sp, nx,
                                           (long long)nx * ny, (long long)nx, (int)nouter, tabs.tw_z.p, inverse, ny,
-                                          (long long)nvox); });
+                                          (long long)nvox, tile_mask(nx, nblk, sz->n * sz->t)); });
       };
       if (axis == 0) fx();
       else if (axis == 1) fy();
@@ -1115,7 +1116,7 @@ struct Solver {
         const long long nblk = (long long)((nx + cz->t - 1) / cz->t) * ny * nb;
         require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
         timed(2, [&] { hipLaunchKernelGGL(cz->fn, dim3((unsigned)nblk), dim3(cz->nt), 0, stream, ws.spec, tb, c,
-                                          tabs.tw_z.p, ws.parity, jj, cv); });
+                                          tabs.tw_z.p, ws.parity, jj, cv, tile_mask(nx, nblk, P * cz->n * cz->t)); });
         return;
       }
       if (dz) {
@@ -1124,7 +1125,7 @@ struct Solver {
         const size_t lds = P == 3 ? dz->lds_green3(rtp[2].da) : dz->lds_strided(rtp[2].da);
         timed(2, [&] { hipLaunchKernelGGL(P == 3 ? dz->strided_green3 : dz->strided_green, dim3((unsigned)nblk),
                                           dim3(dz->nt_strided), lds, stream, ws.spec, tb, c,
-                                          dz->strided_args(rtp[2].da, nx, nblk, P), ws.parity, jj, cv); });
+                                          rtp[2].da, ws.parity, jj, cv, tile_mask(nx, nblk, P * nz * dz->lines)); });
         return;
       }
       if (!bz) {
@@ -1141,7 +1142,7 @@ struct Solver {
       const long long nblk = (long long)((nx + bz->t - 1) / bz->t) * ny * nv;
       require(nblk < (1ll << 31), CBS_ERR_UNSUPPORTED, "z transform batch too large for one launch");
       timed(2, [&] { hipLaunchKernelGGL(bz->strided_green, dim3((unsigned)nblk), dim3(bz->nt), 0, stream, ws.spec,
-                                        tb, c, rtp[2].ba, ws.parity, jj, cv); });
+                                        tb, c, rtp[2].ba, ws.parity, jj, cv, tile_mask(nx, nblk, nz * bz->t)); });
     };
     xpass(UPD_NONE, FWD_P0, 0, 1);
     for (int jj = 1; jj <= M; ++jj) {
@@ -1618,7 +1619,8 @@ struct Solver {
       const int nt = (fx + ffp.st->t - 1) / ffp.st->t;
       require((long long)nt * nf < (1ll << 31), CBS_ERR_UNSUPPORTED, "field transform batch too large for one launch");
       timed(2, [&] { hipLaunchKernelGGL(ffp.st->fn, dim3((unsigned)(nt * nf)), dim3(ffp.st->nt), 0, stream, buf, fx,
-                                        (long long)fx, (long long)fx * fy, (int)nf, ffp.twy.p, inverse, (int)nf, 0ll); });
+                                        (long long)fx, (long long)fx * fy, (int)nf, ffp.twy.p, inverse, (int)nf, 0ll,
+                                        tile_mask(fx, (long long)nt * nf, ffp.st->n * ffp.st->t)); });
     };
     if (!inverse) { rows(); cols(); }
     else { cols(); rows(); }
@@ -1684,7 +1686,8 @@ struct Solver {
       require((long long)nt * nslices < (1ll << 31), CBS_ERR_UNSUPPORTED, "2D FFT batch too large for one launch");
       const dim3 g((unsigned)(nt * nslices));
       timed(2, [&] { hipLaunchKernelGGL(st->fn, g, dim3(st->nt), 0, stream, buf, cx, (long long)cx,
-                                        (long long)cx * cy, (int)nslices, io_tw_cy.p, inverse, (int)nslices, 0ll); });
+                                        (long long)cx * cy, (int)nslices, io_tw_cy.p, inverse, (int)nslices, 0ll,
+                                        tile_mask(cx, (long long)nt * nslices, st->n * st->t)); });
     };
     if (!inverse) { fx_(); fy_(); }
     else { fy_(); fx_(); }
